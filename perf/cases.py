@@ -37,6 +37,12 @@ MODELS = {
 }
 
 
+def _model(case):
+    """The case's model, with a vocabulary of the case's own where it has one (fine-tuned models extend or cut it)."""
+    c = MODELS[case["model"]]
+    return dict(c, vocab=case["vocab"]) if "vocab" in case else c
+
+
 def listed():
     return [
         # one token's q/k/v projections of the smallest model: the smallest call, where latency is all
@@ -83,9 +89,10 @@ def draw(rng):
         m = min(_log_int(rng, 1, 512), max(1, 512 * 14336 * 4096 // (n_in * sum(outs))))
         return dict(kind=kind, type=qt, n_in=n_in, n_outs=",".join(map(str, outs)), m=m, bias=rng.random() < 0.3)
     if kind == "step":
-        return dict(kind=kind, model="smollm2-135m", layers=rng.randint(4, 29))
+        return dict(kind=kind, model="smollm2-135m", layers=rng.randint(4, 29), vocab=_log_int(rng, 8000, 49152))
     if kind == "logits":
-        return dict(kind=kind, model=rng.choice(sorted(MODELS)), m=rng.randint(1, 8))
+        c = rng.choice(sorted(MODELS))
+        return dict(kind=kind, model=c, m=rng.randint(1, 8), vocab=_log_int(rng, 8000, MODELS[c]["vocab"]))
     if kind == "sample":
         return dict(kind=kind, n=_log_int(rng, 32000, 262144), temperature=round(rng.uniform(0.5, 1.3), 3),
                     top_p=rng.choice([0.5, 0.8, 0.9, 0.95, 1.0]))
@@ -171,7 +178,7 @@ def prepare(case, seed):
                     bias=[0.1 * _normal((r,), g) for r in outs] if case["bias"] else None,
                     x=_activations(case["m"], case["n_in"], g))
     if kind == "layer":
-        c, m = MODELS[case["model"]], case["m"]
+        c, m = _model(case), case["m"]
         gate = _normal((m, c["ffn"]), g)
         return dict(case=case, c=c, w=_layer_weights(c, g), x=_activations(m, c["hidden"], g),
                     attn=0.3 * _normal((m, c["qdim"]), g), mid=_activations(m, c["hidden"], g),
@@ -179,7 +186,7 @@ def prepare(case, seed):
     if kind == "step":
         return _prepare_step(case, g)
     if kind == "logits":
-        c = MODELS[case["model"]]
+        c = _model(case)
         return dict(case=case, c=c, w=_weights(c["logits"], c["vocab"], c["hidden"], g),
                     hidden=_normal((case["m"], c["hidden"]), g))
     if kind == "sample":
@@ -194,7 +201,7 @@ def prepare(case, seed):
 
 def _prepare_step(case, g):
     """The decode step captured once in a HIP graph, as a serving loop keeps it."""
-    c = MODELS[case["model"]]
+    c = _model(case)
     s = dict(case=case, c=c, layers=[_layer_weights(c, g) for _ in range(case["layers"])],
              embd=_weights(c["logits"], c["vocab"], c["hidden"], g),  # tied: also the output matrix
              norm=1 + 0.1 * _normal((c["hidden"],), g),
@@ -276,7 +283,7 @@ def work(case):
         parts = [_linear_work(case["type"], int(r), case["n_in"], case["m"]) for r in case["n_outs"].split(",")]
         return {"bytes": sum(p[0] for p in parts) + 4 * case["m"] * case["n_in"], "flops": sum(p[1] for p in parts)}
     if kind in ("layer", "step"):
-        c, m = MODELS[case["model"]], case.get("m", 1)
+        c, m = _model(case), case.get("m", 1)
         parts = {k: _linear_work(*v, m) for k, v in _layer_shapes(c).items()}
         # gate and up leave as their product
         b = sum(p[0] for p in parts.values()) - 4 * m * c["ffn"] + 8 * c["hidden"]
@@ -286,7 +293,7 @@ def work(case):
         lb, lf = _linear_work(c["logits"], c["vocab"], c["hidden"], 1)
         return {"bytes": case["layers"] * b + lb, "flops": case["layers"] * f + lf}
     if kind == "logits":
-        c, m = MODELS[case["model"]], case["m"]
+        c, m = _model(case), case["m"]
         b, f = _linear_work(c["logits"], c["vocab"], c["hidden"], m)
         return {"bytes": b + 4 * m * c["hidden"], "flops": f}
     if kind == "sample":
