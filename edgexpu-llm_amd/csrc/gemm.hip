@@ -97,14 +97,8 @@ constexpr int kPackF32Tokens = 4;  // tokens per wavefront of the f32 pack
 // everything in registers.  The 16 lanes 16 t4 + 4 j + q of token t4 hold
 // its elements 64 j + 8 q .. + 7 and 64 j + 32 + 8 q .. + 7: the code vectors
 // of K-steps 2 q and 2 q + 1 of half j & 1, lane half j >> 1, with no
-// exchange.  The Q8_K quantization (src/gguf_dot_q8.c:360-412) runs over a
-// 16-lane row: the largest |x| (zeros and NaN never enter) by a row max,
-// then iscale = -127 / max|x| and each code as quantize_q8_k_kernel forms
-// it.  The reference's max carries the sign of the first element of largest
-// |x|; where that is negative, this block is the reference's with codes,
-// bsums and d negated, which every product of the GEMM, dx * (C d - mn dmin)
-// with C and mn integer sums of the codes, leaves word for word (sum |q| is
-// the same either way).
+// exchange; the Q8_K quantization (src/gguf_dot_q8.c:360-412) runs over a
+// 16-lane row (q8k_quantize_row16).
 __global__ __launch_bounds__(kPackThreads) void q8k_pack_f32_kernel(const float *__restrict__ x, int ldx, int m,
                                                                     int K, int ntb, uint8_t *__restrict__ pack) {
     const int nb = K / kQKK;
@@ -131,42 +125,8 @@ __global__ __launch_bounds__(kPackThreads) void q8k_pack_f32_kernel(const float 
             xs[4 * k + 3] = v[k].w;
         }
     }
-    uint32_t bb[16], amax_bits = 0u;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float av = fabsf(xs[i]);
-        bb[i] = av > 0.0f ? __float_as_uint(av) : 0u;  // non-negative floats order as their bits
-        amax_bits = max(amax_bits, bb[i]);
-    }
-    amax_bits = row16_max_u32(amax_bits);
-    const bool zero = amax_bits == 0u;
-    const float iscale = -127.0f / __uint_as_float(amax_bits);
-    int qv[16], lo8 = 0, hi8 = 0, sq = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float pv = iscale * xs[i];
-        // lrintf: a NaN or infinite product gives LONG_MIN, whose low 32 bits are 0
-        int c = fabsf(pv) < 2147483648.0f ? (int)rintf(pv) : 0;
-        c = c > 127 ? 127 : (c < -127 ? -127 : c);
-        c = zero ? 0 : c;
-        qv[i] = c;
-        if (i < 8)
-            lo8 += c;
-        else
-            hi8 += c;
-        sq += abs(c);
-    }
-    const float d = zero ? 0.0f : 1.0f / iscale;
-    // bsums: lanes q and q ^ 1 share the 16-element groups 4 j + q / 2 (low)
-    // and 4 j + 2 + q / 2 (high); lane q = 0 then takes groups 4 j + 1 and
-    // 4 j + 3 from lane q = 2
-    lo8 += (int)dpp_u32<kDppXor1>((uint32_t)lo8);
-    hi8 += (int)dpp_u32<kDppXor1>((uint32_t)hi8);
-    const int lo_n = (int)dpp_u32<kDppXor2>((uint32_t)lo8), hi_n = (int)dpp_u32<kDppXor2>((uint32_t)hi8);
-    sq += (int)dpp_u32<kDppXor1>((uint32_t)sq);
-    sq += (int)dpp_u32<kDppXor2>((uint32_t)sq);
-    sq += (int)dpp_u32<kDppHalfMirror>((uint32_t)sq);
-    sq += (int)dpp_u32<kDppMirror>((uint32_t)sq);
+    int qv[16];
+    const Q8KRow16 k = q8k_quantize_row16(xs, qv);
 
     const int tb = t / kTokB, tt = (t % kTokB) / 32, tl = t % 32;
     const int h = j >> 1, hf = j & 1;
@@ -185,13 +145,13 @@ __global__ __launch_bounds__(kPackThreads) void q8k_pack_f32_kernel(const float 
     // row's groups 4 j .. 4 j + 3 are its bytes 8 hf .. 8 hf + 7
     if (q == 0) {
         uint2 o;
-        o.x = h2_bits(lo8, lo_n);
-        o.y = h2_bits(hi8, hi_n);
+        o.x = h2_bits(k.lo, k.lo_next);
+        o.y = h2_bits(k.hi, k.hi_next);
         *reinterpret_cast<uint2 *>(blk + kPkCodes + tt * 1024 + (tl + 32 * h) * 16 + 8 * hf) = o;
     }
     if (r == 0) {
-        *reinterpret_cast<float *>(blk + kPkCodes + kPkMn + 4 * (32 * tt + tl)) = d;
-        *reinterpret_cast<int *>(blk + kPkCodes + kPkMn + kPkDx + 4 * (32 * tt + tl)) = sq;
+        *reinterpret_cast<float *>(blk + kPkCodes + kPkMn + 4 * (32 * tt + tl)) = k.d;
+        *reinterpret_cast<int *>(blk + kPkCodes + kPkMn + kPkDx + 4 * (32 * tt + tl)) = k.sq;
     }
 }
 

@@ -1,0 +1,7 @@
+// Activation-pack geometry of the few-token GEMM (gemm_small.hip).
+#pragma once
+
+namespace exq {
+constexpr int kSmPackK = 4096 + 512 + 64;  // codes, 16-element sums, scales of (super-block, 16 tokens)
+constexpr int kSmPack0 = 512 + 64;         // codes and scales of (32-element block, 16 tokens)
+}  // namespace exq

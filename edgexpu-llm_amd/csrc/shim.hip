@@ -59,6 +59,14 @@ hipError_t launch_g32_pack(const float *x, const uint8_t *xq, size_t xq_stride, 
                            hipStream_t st);
 hipError_t launch_gemm_g32(int type, const uint8_t *rw, int n_out, int K, int m, const uint8_t *pack, float *part,
                            unsigned *cnt, const float *bias, float *out, int ldo, hipStream_t st);
+size_t gemm_small_pack_bytes(int type, int m, int K);
+hipError_t launch_small_pack(int type, const float *x, const float *y, float eps, int pro, int m, int K,
+                             uint8_t *pack, hipStream_t st);
+hipError_t launch_small_pack_blocks(int type, const uint8_t *xq, size_t xq_stride, int m, int K, uint8_t *pack,
+                                    hipStream_t st);
+hipError_t launch_gemm_small(int type, int nmat, const uint8_t *const *w, const int *n_out, const float *const *bias,
+                             const float *const *resid, float *const *out, bool pair, size_t row_bytes, int K, int m,
+                             const uint8_t *pack, hipStream_t st);
 bool gemv_fused_supported(int type, int K, int m);
 bool gemv_fused_f32_supported(int type, int K);
 bool gemv_fused_pro_supported(int type, int K, int pro);
@@ -125,6 +133,8 @@ struct State {
     void *lws = nullptr;    // layer entry: prologue activation and pre-residual outputs
     size_t lws_cap = 0;
     int prefill_mode = 0;   // EDGEXPU_HIP_PREFILL_EXACT_INT8 / _F16
+    void *tws = nullptr;    // few-token GEMM: activation pack
+    size_t tws_cap = 0;
     void *gws = nullptr;    // exact prefill GEMM: activation pack
     size_t gws_cap = 0;
     size_t dbuf_cap = 0;
@@ -326,6 +336,24 @@ void *gemm_ws(size_t bytes) {
     return g.gws;
 }
 
+// Workspace of the few-token GEMM (the activation pack), grown on demand.  It
+// starts at 4 MiB, above the pack of 128 tokens of 14336 elements (2.5 MB), so
+// that a step captured in a graph keeps its address whatever prefill sizes
+// run beside it.
+void *small_ws(size_t bytes) {
+    if (bytes <= g.tws_cap) return g.tws;
+    if (g.tws != nullptr) {
+        if (!hip_ok(hipDeviceSynchronize(), "few-token workspace sync")) return nullptr;
+        (void)hipFree(g.tws);
+        g.tws = nullptr;
+        g.tws_cap = 0;
+    }
+    const size_t cap = align_up(bytes, (size_t)4 << 20);
+    if (!hip_ok(hipMalloc(&g.tws, cap), "hipMalloc few-token workspace")) return nullptr;
+    g.tws_cap = cap;
+    return g.tws;
+}
+
 // Formats with an exact matrix-core prefill GEMM: Q4_K straight from its
 // blocks (gemm.hip), Q5_K and Q6_K over a per-call repack (gemm_kq.hip), and
 // Q8_0 / Q4_0 / Q5_0 over a per-call repack against Q8_0 activations
@@ -405,6 +433,54 @@ bool run_gemm_exact(uint32_t type, int nmat, const void *const *w, const int *n_
 bool use_exact_gemm(uint32_t type, int nmat, const void *const *w, const int *n_out, int n_in, int m) {
     return m >= gemm_min_tokens(type) && g.prefill_mode == EDGEXPU_HIP_PREFILL_EXACT_INT8 &&
            exact_gemm_type(type, nmat, w, n_out, n_in, m);
+}
+
+// The few-token GEMM (gemm_small.hip) takes Q4_K (rows of 16-byte vectors),
+// Q6_K and Q8_0 products of kSmallMinTokens to kSmallMaxTokens tokens.
+constexpr int kSmallMinTokens = 5;
+constexpr int kSmallMaxTokens = 64;
+bool use_small(uint32_t type, int nmat, const void *const *w, int m) {
+    static const int lo = tuning_knob("EXQ_SM_LO", kSmallMinTokens), hi = tuning_knob("EXQ_SM_HI", kSmallMaxTokens);
+    if (m < lo || m > hi) return false;
+    if (type == (uint32_t)kTypeQ8_0 || type == (uint32_t)kTypeQ6_K) return true;
+    if (type != (uint32_t)kTypeQ4_K) return false;
+    if (m >= gemm_min_tokens(type) && g.prefill_mode != EDGEXPU_HIP_PREFILL_EXACT_INT8) return false;
+    for (int z = 0; z < nmat; ++z)
+        if (!aligned16(w[z])) return false;
+    return true;
+}
+
+// One pack launch (f32 activations through prologue pro: 1 RMSNorm with
+// weight y, 2 silu(x) * y, 0 none; or quantized blocks xq), then one launch
+// over all the matrices.
+bool run_small(uint32_t type, int nmat, const void *const *w, const int *n_out, const float *const *bias,
+               const float *const *resid, float *const *out, bool pair, const float *x, const float *y, float eps,
+               int pro, const uint8_t *xq, size_t xq_stride, int m, int n_in, hipStream_t st) {
+    uint8_t *pack = (uint8_t *)small_ws(gemm_small_pack_bytes((int)type, m, n_in));
+    if (pack == nullptr) return false;
+    const hipError_t e = x != nullptr ? launch_small_pack((int)type, x, y, eps, pro, m, n_in, pack, st)
+                                      : launch_small_pack_blocks((int)type, xq, xq_stride, m, n_in, pack, st);
+    return hip_ok(e, "pack activations") &&
+           hip_ok(launch_gemm_small((int)type, nmat, (const uint8_t *const *)w, n_out, bias, resid, out, pair,
+                                    edgexpu_hip_row_bytes(type, n_in), n_in, m, pack, st),
+                  "gemm_small");
+}
+
+// True when writing the outputs element by element could be seen through a
+// residual or bias still to be read: some output overlaps a residual (other
+// than its own, exactly) or a bias.
+bool outputs_overlap(int nmat, float *const *out, const float *const *resid, const float *const *bias,
+                     const int *n_out, int m) {
+    const auto cross = [](const float *a, size_t na, const float *b, size_t nb) {
+        return b != nullptr && (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+    };
+    for (int z = 0; z < nmat; ++z)
+        for (int y = 0; y < nmat; ++y) {
+            const size_t nz = (size_t)m * n_out[z], ny = (size_t)m * n_out[y];
+            if (resid != nullptr && !(y == z && resid[y] == out[z]) && cross(out[z], nz, resid[y], ny)) return true;
+            if (bias != nullptr && cross(out[z], nz, bias[y], (size_t)n_out[y])) return true;
+        }
+    return false;
 }
 
 // Workspace carve-up for m tokens of K elements.
@@ -520,6 +596,9 @@ bool run_q8_product(uint32_t type, const void *w, int n_out, int n_in, int m, co
                     float *out, int ldo, hipStream_t st) {
     const size_t rb = edgexpu_hip_row_bytes(type, n_in);
     const size_t ab = act_bytes(type, n_in);
+    if (ldo == n_out && use_small(type, 1, &w, m))
+        return run_small(type, 1, &w, &n_out, &bias, nullptr, &out, false, nullptr, nullptr, 0.0f, 0, xq, ab, m, n_in,
+                         st);
     if (m >= gemm_min_tokens(type) && exact_gemm_type(type, 1, &w, &n_out, n_in, m)) {
         if (g.prefill_mode == EDGEXPU_HIP_PREFILL_F16 && gemm_q8_supported((int)type, n_out, n_in, m)) {
             void *ws = f16ws(gemm_f16_workspace(m, n_out, n_in));
@@ -562,6 +641,8 @@ bool run_linear_group(uint32_t type, int nmat, const void *const *w, const int *
                 return false;
         return true;
     }
+    if (use_small(type, nmat, w, m))
+        return run_small(type, nmat, w, n_out, bias, nullptr, out, false, x, nullptr, 0.0f, 0, nullptr, 0, m, n_in, st);
     // two to four tokens of the rows the streaming GEMV takes are quantized
     // inside its workgroups too; other long rows quantize once in their own
     // launch
@@ -641,6 +722,7 @@ void edgexpu_hip_shutdown(void) {
     if (g.sws) (void)hipFree(g.sws);
     if (g.lws) (void)hipFree(g.lws);
     if (g.gws) (void)hipFree(g.gws);
+    if (g.tws) (void)hipFree(g.tws);
     (void)hipStreamDestroy(g.stream);
     const int err = g.err;
     char msg[sizeof(g.msg)];
@@ -881,6 +963,12 @@ int edgexpu_hip_layer_linear_dev(int nmat, float *const *out, const float *x, co
                       "layer_linear fused")
                    ? 1
                    : 0;
+    // a few tokens: the prologue in the pack, the residual in the product's store
+    if (use_small(type, nmat, w, m) && !outputs_overlap(nmat, out, residual, bias, n_out, m))
+        return run_small(type, nmat, w, n_out, bias, residual, out, false, x, pro == 1 ? norm_weight : x2, eps, pro,
+                         nullptr, 0, m, n_in, st)
+                   ? 1
+                   : 0;
     // otherwise the same arithmetic in steps: prologue kernel, projection,
     // residual add (the projection writes to the workspace first, so out may
     // be the residual)
@@ -943,6 +1031,13 @@ int edgexpu_hip_gate_up_silu_dev(float *act, const float *x, const float *norm_w
                    ? 1
                    : 0;
     }
+    float *act_out[2] = {act, nullptr};
+    if (use_small(type, 2, wg, m) && !outputs_overlap(1, act_out, nullptr, bg, nn, m) &&
+        !outputs_overlap(1, act_out, nullptr, bg + 1, nn, m))
+        return run_small(type, 2, wg, nn, bg, nullptr, act_out, true, x, norm_weight, eps, pro, nullptr, 0, m, n_in,
+                         st)
+                   ? 1
+                   : 0;
     // otherwise: the RMSNorm, gate and up into one sizing of the layer
     // workspace (nothing below grows it), then silu * up
     const size_t nf = align_up((size_t)m * n_ff, 64), ni = pro != 0 ? align_up((size_t)m * n_in, 64) : 0;

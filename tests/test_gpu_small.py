@@ -1,0 +1,117 @@
+"""Products of 5 to 64 tokens (csrc/gemm_small.hip) against the oracle.
+
+Q4_K, Q6_K and Q8_0 rows on the integer matrix cores, 16 rows by up to 64
+tokens per workgroup with K split over its waves: every output within 1e-5 of
+its conditioning scale (the block integers are exact; what differs from the
+oracle is the order of the f32 sum over blocks), at the edges of the token
+tiles (16), the row tiles (16, 32), the K units (one super-block, one 32-element
+block, counts that do not divide the waves) and the wave counts (1 to 16).
+"""
+import numpy as np
+import pytest
+import torch
+
+import edgexpu_amd as E
+import npref
+from edgexpu_amd import synth
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+
+
+def bits(a):
+    return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+
+
+def quantize(ora, qt, x):
+    return np.stack([(ora.quantize_q8_0 if qt == 8 else ora.quantize_q8_k)(r) for r in x])
+
+
+def scales(qt, w, xq):
+    """S[t][i] of the integer dot (float64)."""
+    return np.stack([[npref.q8_dot_f64(qt, r, q)[1] for r in w] for q in xq])
+
+
+@pytest.mark.parametrize("qt,n_in", [(12, 256), (12, 2560), (12, 4352), (14, 256), (14, 2816), (14, 9728), (8, 32),
+                                     (8, 576), (8, 2080)])
+@pytest.mark.parametrize("m", [5, 16, 17, 33, 64])
+def test_small_vs_oracle(hipdev, ora, qt, n_in, m):
+    """A group of ragged row counts (one below a tile, one past it, one row),
+    with and without bias; equal to the call of each matrix alone and to the
+    call over quantized blocks bit for bit."""
+    n_outs = (15, 33, 1)
+    rng = np.random.default_rng(100 * qt + n_in + m)
+    ws = [synth.np_weights(qt, n, n_in, rng) for n in n_outs]
+    x = synth.np_activations(m, n_in, rng)
+    biases = [rng.normal(0, 0.3, n).astype(np.float32) if z != 1 else None for z, n in enumerate(n_outs)]
+    wd, xd = [dev(w) for w in ws], dev(x)
+    bd = [None if b is None else dev(b) for b in biases]
+    outs = E.linear_quant_group(wd, qt, xd, list(n_outs), n_in, biases=bd)
+    xq = quantize(ora, qt, x)
+    for z, n in enumerate(n_outs):
+        got = outs[z].cpu().numpy()
+        want = ora.linear_quant_batch(x, ws[z], qt, biases[z], m, n, n_in)
+        S = scales(qt, ws[z], xq) + (0 if biases[z] is None else np.abs(biases[z])[None, :])
+        assert np.all(np.abs(got - want) <= TOL * S), f"matrix {z}"
+        one = E.linear_quant_batch(wd[z], qt, xd, n, n_in, bias=bd[z]).cpu().numpy()
+        assert np.array_equal(bits(got), bits(one)), f"matrix {z} alone"
+        blk = E.gemv_q8(wd[z], qt, dev(xq), m, n, n_in, bias=bd[z]).cpu().numpy()
+        assert np.array_equal(bits(got), bits(blk)), f"matrix {z} from blocks"
+
+
+@pytest.mark.parametrize("qt,n_in,n_out", [(12, 4096, 8200), (14, 2560, 300), (8, 576, 100)])
+@pytest.mark.parametrize("m", [7, 40])
+def test_small_layer_calls_equal_the_steps(hipdev, qt, n_in, n_out, m):
+    """RMSNorm and SiLU-mul in the pack, the residual in the store (also over
+    itself) and the gate / up pair: equal to the separate device calls bit for
+    bit.  An output that overlaps another matrix's residual takes the steps,
+    where every product is complete before a residual is read."""
+    rng = np.random.default_rng(qt + n_in + m)
+    w, w2 = (dev(synth.np_weights(qt, n_out, n_in, rng)) for _ in range(2))
+    x, y = (dev(rng.normal(0, 1, (m, n_in)).astype(np.float32)) for _ in range(2))
+    nw = dev(rng.normal(1, 0.2, n_in).astype(np.float32))
+    b, b2 = (dev(rng.normal(0, 0.5, n_out).astype(np.float32)) for _ in range(2))
+    res = dev(rng.normal(0, 4, (m, n_out)).astype(np.float32))
+
+    def eq(a, c):
+        assert np.array_equal(bits(a.cpu().numpy()), bits(c.cpu().numpy()))
+
+    lin = lambda a, ww, bb: E.linear_quant_batch(ww, qt, a, n_out, n_in, bias=bb)  # noqa: E731
+    norm = E.rmsnorm(x, nw, 1e-5)
+    r = res.clone()
+    E.layer_linear([w], qt, x, (n_out,), n_in, norm_weight=nw, biases=[b], residuals=[r], outs=[r])
+    eq(r, E.add(res, lin(norm, w, b)))
+    got, = E.layer_linear([w], qt, x, (n_out,), n_in, x2=y, residuals=[res])
+    eq(got, E.add(res, lin(E.silu_mul(x, y), w, None)))
+    act = E.gate_up_silu(w, w2, qt, x, n_out, n_in, norm_weight=nw, b_gate=b, b_up=b2)
+    eq(act, E.silu_mul(lin(norm, w, b), lin(norm, w2, b2)))
+    # out 0 is matrix 1's residual
+    o0, o1 = res.clone(), torch.empty_like(res)
+    E.layer_linear([w, w2], qt, x, (n_out, n_out), n_in, residuals=[res, o0], outs=[o0, o1])
+    eq(o0, E.add(res, lin(x, w, None)))
+    eq(o1, E.add(o0, lin(x, w2, None)))
+
+
+@pytest.mark.parametrize("qt,n_in", [(12, 2560), (14, 2560), (8, 576)])
+def test_small_special_activations(hipdev, ora, qt, n_in):
+    """Tokens holding zeros, infinities and NaN: finite tokens beside them are
+    untouched, and each output is finite exactly where the one-token call's is."""
+    m, n_out = 9, 40
+    rng = np.random.default_rng(qt)
+    w = synth.np_weights(qt, n_out, n_in, rng)
+    x = synth.np_activations(m, n_in, rng)
+    x[1] = 0.0
+    x[3, 5] = np.inf
+    x[4, 300] = np.nan
+    x[6, :40] = 1e-40
+    got = E.linear_quant_batch(dev(w), qt, dev(x), n_out, n_in).cpu().numpy()
+    for t in range(m):
+        one = E.linear_quant_batch(dev(w), qt, dev(x[t:t + 1]), n_out, n_in).cpu().numpy()[0]
+        assert np.array_equal(np.isfinite(got[t]), np.isfinite(one)), t
+    fin = np.isfinite(x).all(axis=1)
+    want = ora.linear_quant_batch(x[fin], w, qt, None, int(fin.sum()), n_out, n_in)
+    assert np.all(np.abs(got[fin] - want) <= TOL * scales(qt, w, quantize(ora, qt, x[fin])))
