@@ -69,12 +69,14 @@ __device__ __forceinline__ int piece_of(int g) { return ((g & 1) << 1) | (g >> 1
 //         64 j + 8 piece(g) .. + 7 and 64 j + 32 + 8 piece(g) .. + 7
 //   bsums [lane 64][4 fp16]     lane t + 16 g: 16-element sums 4 g .. 4 g + 3
 //   dx    [16] f32
-// Q8_0 pack, kSmPack0 bytes per (32-element block, tile):
-//   codes [lane 64][8 B]        lane t + 16 g: elements 8 g .. 8 g + 7
-//   dx    [16] f32
+// Q8_0 pack, kSmPack0 bytes per (pair of 32-element blocks, tile):
+//   codes [lane 64][16 B]       lane t + 16 g: elements 8 piece(g) .. + 7 of
+//         the even and of the odd block
+//   dx    [2][16] f32
+// (an odd last block leaves its partner's places unwritten, and unread).
 // Tokens of a tile past m are not written: a token's column of the product
 // touches no other, and theirs is never stored.
-constexpr int kSmBs = 4096, kSmDx = 4608;
+constexpr int kSmBs = 4096, kSmDx = 4608, kSmDx0 = 1024;
 
 // The prologue of one value: RMSNorm (x * scale) * w, silu(x) * x2, or x.
 template <int PRO>
@@ -241,10 +243,13 @@ __global__ __launch_bounds__(1024) void small_pack_0_kernel(const float *__restr
             const int k = (v >= -2147483648.0f && v < 2147483648.0f) ? (int)v : INT32_MIN;
             qv[i] = k < -128 ? -128 : (k > 127 ? 127 : k);
         }
-        uint8_t *blk = pack + ((size_t)b * ntt + (t >> 4)) * kSmPack0;
-        const int tl = t & 15;
-        *reinterpret_cast<uint2 *>(blk + (tl + 16 * g) * 8) = make_uint2(bytes4(qv), bytes4(qv + 4));
-        if (g == 0) *reinterpret_cast<float *>(blk + 512 + 4 * tl) = f16_bits_to_f32(f32_to_f16_rne(amax / 127.0f));
+        uint8_t *blk = pack + ((size_t)(b >> 1) * ntt + (t >> 4)) * kSmPack0;
+        const int tl = t & 15, odd = b & 1;
+        *reinterpret_cast<uint2 *>(blk + (tl + 16 * piece_of(g)) * 16 + 8 * odd) =
+            make_uint2(bytes4(qv), bytes4(qv + 4));
+        if (g == 0)
+            *reinterpret_cast<float *>(blk + kSmDx0 + 4 * (16 * odd + tl)) =
+                f16_bits_to_f32(f32_to_f16_rne(amax / 127.0f));
     }
 }
 
@@ -256,11 +261,11 @@ __global__ __launch_bounds__(256) void small_pack_0_blocks_kernel(const uint8_t 
     const int b = (int)blockIdx.y * 64 + (int)(threadIdx.x >> 2);
     if (b >= nb) return;
     const uint8_t *src = xq + (size_t)t * xq_stride + (size_t)b * kBytesQ8_0;
-    uint8_t *blk = pack + ((size_t)b * ntt + (t >> 4)) * kSmPack0;
-    const int tl = t & 15;
-    *reinterpret_cast<uint2 *>(blk + (tl + 16 * g) * 8) = ldg8(src + 2 + 8 * g);
+    uint8_t *blk = pack + ((size_t)(b >> 1) * ntt + (t >> 4)) * kSmPack0;
+    const int tl = t & 15, odd = b & 1;
+    *reinterpret_cast<uint2 *>(blk + (tl + 16 * piece_of(g)) * 16 + 8 * odd) = ldg8(src + 2 + 8 * g);
     if (g == 0)
-        *reinterpret_cast<float *>(blk + 512 + 4 * tl) = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(src));
+        *reinterpret_cast<float *>(blk + kSmDx0 + 4 * (16 * odd + tl)) = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(src));
 }
 
 // --------------------------------------------------------------- formats
@@ -320,13 +325,14 @@ struct SmallQ4K {
         o.d = f16_bits_to_f32(w.hd.x & 0xffffu);
         o.nd = -f16_bits_to_f32(w.hd.x >> 16);
     }
-    __device__ static __forceinline__ void load_a(A &a, const uint8_t *blk, int, int lane) {
+    __device__ static __forceinline__ void load_a(A &a, const uint8_t *pk, int u, int, int ntt, int tt, int lane) {
+        const uint8_t *blk = pk + ((size_t)u * ntt + tt) * kSmPackK;
 #pragma unroll
         for (int j = 0; j < 4; ++j) a.c[j] = *reinterpret_cast<const uint4 *>(blk + j * 1024 + lane * 16);
         a.bs = __builtin_bit_cast(v4h, *reinterpret_cast<const uint2 *>(blk + kSmBs + lane * 8));
         a.dx = *reinterpret_cast<const float4 *>(blk + kSmDx + 16 * (lane >> 4));
     }
-    __device__ static __forceinline__ void dot(float (&acc)[4], const A &a, const Op &o, int) {
+    __device__ static __forceinline__ void dot(float (&acc)[4], const A &a, const Op &o, int, int, int) {
         int s[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -415,10 +421,11 @@ struct SmallQ6K {
         for (int i = 0; i < 4; ++i) o.mn[i] = (_Float16)(float)(int8_t)((sg >> (8 * i)) & 0xffu);
         o.d = f16_bits_to_f32(w.d);
     }
-    __device__ static __forceinline__ void load_a(A &a, const uint8_t *blk, int u, int lane) {
-        SmallQ4K::load_a(a, blk, u, lane);
+    __device__ static __forceinline__ void load_a(A &a, const uint8_t *pk, int u, int end, int ntt, int tt,
+                                                  int lane) {
+        SmallQ4K::load_a(a, pk, u, end, ntt, tt, lane);
     }
-    __device__ static __forceinline__ void dot(float (&acc)[4], const A &a, const Op &o, int g) {
+    __device__ static __forceinline__ void dot(float (&acc)[4], const A &a, const Op &o, int, int, int g) {
         const uint32_t first = (g & 1) ? 0u : ~0u;
         int s[4] = {0, 0, 0, 0};
 #pragma unroll
@@ -438,94 +445,122 @@ struct SmallQ6K {
     }
 };
 
-// Q8_0: a step takes up to four 32-element blocks (a block alone is one
-// product behind three loads), those past the wave's range with scale 0.
+// Q8_0: a step takes two pairs of 32-element blocks.  Of a pair, lane groups
+// 0 and 1 read the halves of the even block's codes and groups 2 and 3 those
+// of the odd block's, and v_permlane32_swap deals them out as for Q4_K; group
+// g reads the scale of block g of the step, and a lane takes the four of its
+// row from there.  Five loads per step for 2176 bytes of 16 rows; an 8-byte
+// load and a scale per block and lane were twelve, which bounded it (8 tokens
+// of 14336 rows of 4096: 56 us).
 struct SmallQ80 {
     static constexpr int kType = kTypeQ8_0;
     static constexpr int kUnits = 4;
     struct W {
-        uint2 q[4];
-        uint32_t d[4];
+        uint4 q[2];
+        uint32_t d;
     };
     struct Op {
-        uint2 q[4];
+        uint32_t q[4][2];
         float d[4];
     };
     struct A {
-        uint2 c[4];
+        uint4 c[2];
         float4 dx[4];
     };
     __device__ static __forceinline__ void load_w(W &w, const uint8_t *row, int u, int end, int g) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint8_t *p = row + (size_t)min(u + i, end - 1) * kBytesQ8_0;
-            w.q[i] = ldg8_a2(p + 2 + 8 * g);
-            w.d[i] = u + i < end ? *reinterpret_cast<const uint16_t *>(p) : 0u;
-        }
+        for (int i = 0; i < 2; ++i)
+            w.q[i] = ldg16_a2(row + (size_t)min(u + 2 * i + (g >> 1), end - 1) * kBytesQ8_0 + 2 + 16 * (g & 1));
+        w.d = *reinterpret_cast<const uint16_t *>(row + (size_t)min(u + g, end - 1) * kBytesQ8_0);
     }
     __device__ static __forceinline__ void decode(Op &o, const W &w, int) {
+        const int r16 = threadIdx.x & 15;
+        const float d = f16_bits_to_f32(w.d);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const auto x = __builtin_amdgcn_permlane32_swap(w.q[i].x, w.q[i].z, false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(w.q[i].y, w.q[i].w, false, false);
+            o.q[2 * i][0] = (uint32_t)x[0];
+            o.q[2 * i][1] = (uint32_t)y[0];
+            o.q[2 * i + 1][0] = (uint32_t)x[1];
+            o.q[2 * i + 1][1] = (uint32_t)y[1];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o.d[i] = __shfl(d, r16 + 16 * i, 64);
+    }
+    __device__ static __forceinline__ void load_a(A &a, const uint8_t *pk, int u, int end, int ntt, int tt, int lane) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint8_t *blk = pk + ((size_t)(min(u + 2 * i, end - 1) >> 1) * ntt + tt) * kSmPack0;
+            a.c[i] = *reinterpret_cast<const uint4 *>(blk + lane * 16);
+            a.dx[2 * i] = *reinterpret_cast<const float4 *>(blk + kSmDx0 + 16 * (lane >> 4));
+            a.dx[2 * i + 1] = *reinterpret_cast<const float4 *>(blk + kSmDx0 + 64 + 16 * (lane >> 4));
+        }
+    }
+    __device__ static __forceinline__ void dot(float (&acc)[4], const A &a, const Op &o, int u, int end, int) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            o.q[i] = w.q[i];
-            o.d[i] = f16_bits_to_f32(w.d[i]);
+            if (u + i >= end) break;  // wave-uniform
+            const uint4 c = a.c[i >> 1];
+            const v4i p = mfma_i8((i & 1) ? pack2(c.z, c.w) : pack2(c.x, c.y), pack2(o.q[i][0], o.q[i][1]),
+                                  v4i{0, 0, 0, 0});
+            const float dx[4] = {a.dx[i].x, a.dx[i].y, a.dx[i].z, a.dx[i].w};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf((float)p[r] * o.d[i], dx[r], acc[r]);
         }
     }
 };
 
 // --------------------------------------------------------------- product
 
-template <class F>
-struct SmallStep {
-    template <int RT, int TT>
-    __device__ static __forceinline__ void run(float (&acc)[RT][TT][4], const typename F::W (&w)[RT],
-                                               const uint8_t *pk, int u, int, int ntt, int lane) {
-        const int g = lane >> 4;
+// One step of a wave (NEXT: the weights of units un .. are requested too).
+// Loads retire in order: for Q8_0 and Q6_K the token tiles' operands are
+// requested before the next step's weights, so no product waits for those
+// (Q8_0 576 / 1536 layer of 30 tokens 48 us the other way round, 37 us so;
+// Q6_K 9728 down of 64 tokens 38 and 28 us).  Q4_K steps are short of
+// registers instead: holding every operand of more than two tiles halves the
+// waves per CU (gate and up of 64 tokens 54 us), so they take the weights first
+// and the operands tile by tile (48 us).
+template <class F, int RT, int TT, bool NEXT>
+__device__ __forceinline__ void small_step(float (&acc)[RT][TT][4], typename F::W (&w)[RT],
+                                           const uint8_t *const (&row)[RT], const uint8_t *pk, int u, int un, int end,
+                                           int ntt, int lane) {
+    const int g = lane >> 4;
+    typename F::W wn[RT];
+    if constexpr (F::kType != kTypeQ4_K) {
+        typename F::A a[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) F::load_a(a[tt], pk, u, end, ntt, tt, lane);
+        if (NEXT)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) F::load_w(wn[rt], row[rt], un, end, g);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            typename F::Op op;
+            F::decode(op, w[rt], g);
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) F::dot(acc[rt][tt], a[tt], op, u, end, g);
+        }
+    } else {
+        if (NEXT)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) F::load_w(wn[rt], row[rt], un, end, g);
         typename F::Op op[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) F::decode(op[rt], w[rt], g);
-        const uint8_t *blk = pk + (size_t)u * ntt * kSmPackK;
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt) {
             typename F::A a;
-            F::load_a(a, blk + tt * kSmPackK, u, lane);
+            F::load_a(a, pk, u, end, ntt, tt, lane);
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) F::dot(acc[rt][tt], a, op[rt], g);
+            for (int rt = 0; rt < RT; ++rt) F::dot(acc[rt][tt], a, op[rt], u, end, g);
         }
     }
-};
-
-template <>
-struct SmallStep<SmallQ80> {
-    template <int RT, int TT>
-    __device__ static __forceinline__ void run(float (&acc)[RT][TT][4], const SmallQ80::W (&w)[RT], const uint8_t *pk,
-                                               int u, int end, int ntt, int lane) {
-        SmallQ80::Op op[RT];
+    if (NEXT)
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) SmallQ80::decode(op[rt], w[rt], 0);
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-            SmallQ80::A a;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint8_t *blk = pk + ((size_t)min(u + i, end - 1) * ntt + tt) * kSmPack0;
-                a.c[i] = *reinterpret_cast<const uint2 *>(blk + lane * 8);
-                a.dx[i] = *reinterpret_cast<const float4 *>(blk + 512 + 16 * (lane >> 4));
-            }
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (u + i >= end) break;  // wave-uniform
-                    const v4i p = mfma_i8(pack2(a.c[i].x, a.c[i].y), pack2(op[rt].q[i].x, op[rt].q[i].y),
-                                          v4i{0, 0, 0, 0});
-                    const float dx[4] = {a.dx[i].x, a.dx[i].y, a.dx[i].z, a.dx[i].w};
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        acc[rt][tt][r] = __builtin_fmaf((float)p[r] * op[rt].d[i], dx[r], acc[rt][tt][r]);
-                }
-        }
-    }
-};
+        for (int rt = 0; rt < RT; ++rt) w[rt] = wn[rt];
+}
 
 struct SmallArgs {
     const uint8_t *w[4];
@@ -540,12 +575,12 @@ struct SmallArgs {
     int m, ntt;    // tokens, 16-token tiles of the pack
 };
 
-constexpr int kSmSlots = 8;  // waves whose tiles lie in LDS at once
-
-// PAIR: RT = 2, the gate and the up matrix's row tile.
+// PAIR: w[0] and w[1] are gate and up, RT = 2 the row tile of each (two waves
+// of one row tile each would read the operands twice: 31 us against 26 us for
+// 8 tokens of 2 x 14336 rows of 4096).
 template <class F, int RT, int TT, bool PAIR, int MAXW>
 __global__ __launch_bounds__(64 * MAXW) void gemm_small_kernel(SmallArgs a) {
-    __shared__ float4 red[kSmSlots][RT * TT][64];
+    __shared__ float4 red[MAXW][RT * TT][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nw = (int)(blockDim.x >> 6);
@@ -562,7 +597,9 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_small_kernel(SmallArgs a) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
         row[rt] = a.w[PAIR ? rt : z] + (size_t)min(row0 + (PAIR ? 0 : 16 * rt) + r16, n_out - 1) * a.row_bytes;
-    const int k0 = (int)((long long)a.nk * wave / nw), k1 = (int)((long long)a.nk * (wave + 1) / nw);
+    constexpr int kGran = F::kType == kTypeQ8_0 ? 2 : 1;  // Q8_0 blocks go in pairs
+    const int np = (a.nk + kGran - 1) / kGran;
+    const int k0 = kGran * (np * wave / nw), k1 = min(a.nk, kGran * (np * (wave + 1) / nw));
 
     float acc[RT][TT][4];
 #pragma unroll
@@ -578,51 +615,32 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_small_kernel(SmallArgs a) {
         typename F::W w[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) F::load_w(w[rt], row[rt], k0, k1, g);
-        for (int u = k0; u < k1; u += F::kUnits) {
-            typename F::W nw_[RT];
-            const int un = u + F::kUnits < k1 ? u + F::kUnits : u;
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) F::load_w(nw_[rt], row[rt], un, k1, g);
-            SmallStep<F>::template run<RT, TT>(acc, w, pk, u, k1, a.ntt, lane);
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) w[rt] = nw_[rt];
+        // The K-quants' last step requests its own weights again (they hit in
+        // L1): a peeled last step doubles the code, which costs more (Q4_K
+        // down of 64 tokens 38 us against 31 us).  Q8_0's shorter steps peel
+        // it (layer of 8 tokens 40 us unpeeled, 34 us so).
+        if constexpr (F::kUnits == 1) {
+            for (int u = k0; u < k1; ++u)
+                small_step<F, RT, TT, true>(acc, w, row, pk, u, u + 1 < k1 ? u + 1 : u, k1, a.ntt, lane);
+        } else {
+            int u = k0;
+            for (; u + F::kUnits < k1; u += F::kUnits)
+                small_step<F, RT, TT, true>(acc, w, row, pk, u, u + F::kUnits, k1, a.ntt, lane);
+            small_step<F, RT, TT, false>(acc, w, row, pk, u, u, k1, a.ntt, lane);
         }
     }
 
-    // the waves' tiles, added in wave order: waves past the first eight hand
-    // theirs to wave - 8 first
+    // the waves' tiles, added in wave order
 #pragma unroll
-    for (int ph = 0; ph < (MAXW > kSmSlots ? 2 : 1); ++ph) {
-        const bool late = MAXW > kSmSlots && ph == 0;
-        if (late && nw <= kSmSlots) continue;
-        if (late ? wave >= kSmSlots : wave < kSmSlots) {
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int tt = 0; tt < TT; ++tt)
-                    red[wave & (kSmSlots - 1)][rt * TT + tt][lane] =
-                        make_float4(acc[rt][tt][0], acc[rt][tt][1], acc[rt][tt][2], acc[rt][tt][3]);
-        }
-        __syncthreads();
-        if (late) {
-            if (wave + kSmSlots < nw)
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                    for (int tt = 0; tt < TT; ++tt) {
-                        const float4 v = red[wave][rt * TT + tt][lane];
-                        acc[rt][tt][0] += v.x;
-                        acc[rt][tt][1] += v.y;
-                        acc[rt][tt][2] += v.z;
-                        acc[rt][tt][3] += v.w;
-                    }
-            __syncthreads();
-        }
-    }
-    const int ns = min(nw, kSmSlots);
+        for (int tt = 0; tt < TT; ++tt)
+            red[wave][rt * TT + tt][lane] =
+                make_float4(acc[rt][tt][0], acc[rt][tt][1], acc[rt][tt][2], acc[rt][tt][3]);
+    __syncthreads();
     const auto total = [&](int tile_i, int l) {
         float4 s = red[0][tile_i][l];
-        for (int w = 1; w < ns; ++w) {
+        for (int w = 1; w < nw; ++w) {
             const float4 v = red[w][tile_i][l];
             s.x += v.x;
             s.y += v.y;
@@ -666,7 +684,7 @@ using namespace exq;
 
 size_t gemm_small_pack_bytes(int type, int m, int K) {
     const size_t ntt = (size_t)(m + 15) / 16 + 3;  // a launch reads whole groups of up to four tiles
-    return type == kTypeQ8_0 ? (size_t)(K / kQK8_0) * ntt * kSmPack0 : (size_t)(K / kQKK) * ntt * kSmPackK;
+    return type == kTypeQ8_0 ? (size_t)(K / kQK8_0 + 1) / 2 * ntt * kSmPack0 : (size_t)(K / kQKK) * ntt * kSmPackK;
 }
 
 static int small_tiles(int m) { return (m + 15) / 16; }
@@ -723,7 +741,7 @@ static hipError_t small_dispatch(const SmallArgs &a, int rt, int tt, bool pair, 
 #define SM_CASE(T)                                                      \
     case T:                                                             \
         if (pair)                                                       \
-            small_launch<F, 2, T, true>(a, tiles, nw, st);              \
+            small_launch<F, (2), T, true>(a, tiles, nw, st); \
         else if (rt == 2)                                               \
             small_launch<F, 2, T, false>(a, tiles, nw, st);             \
         else                                                            \

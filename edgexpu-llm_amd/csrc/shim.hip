@@ -336,10 +336,9 @@ void *gemm_ws(size_t bytes) {
     return g.gws;
 }
 
-// Workspace of the few-token GEMM (the activation pack), grown on demand.  It
-// starts at 4 MiB, above the pack of 128 tokens of 14336 elements (2.5 MB), so
-// that a step captured in a graph keeps its address whatever prefill sizes
-// run beside it.
+// Workspace of the few-token GEMM (the activation pack), grown on demand in
+// steps of 4 MiB (the pack of 200 tokens of 14336 elements), so that a step
+// captured in a graph keeps its address whatever sizes run beside it.
 void *small_ws(size_t bytes) {
     if (bytes <= g.tws_cap) return g.tws;
     if (g.tws != nullptr) {
@@ -436,14 +435,32 @@ bool use_exact_gemm(uint32_t type, int nmat, const void *const *w, const int *n_
 }
 
 // The few-token GEMM (gemm_small.hip) takes Q4_K (rows of 16-byte vectors),
-// Q6_K and Q8_0 products of kSmallMinTokens to kSmallMaxTokens tokens.
+// Q6_K and Q8_0 products from kSmallMinTokens tokens: up to 64 always, beyond
+// that while rows x K x (64-token blocks, each of which reads the weights
+// again) stays below the line where the 128-token tiles of the prefill GEMMs
+// catch up.  Measured, few-token / prefill, one matrix: Q4_K 4096 x 4096 of
+// 512 tokens (134 M) 48 / 53 us, 4096 x 14336 of 128 (117 M) 50 / 49, 2560 x
+// 9728 of 256 (100 M) 52 / 48; Q6_K 9728 x 2560 of 128 (50 M) 49 / 52, of 256
+// (100 M) 70 / 62, 2560 x 2560 of 512 (8 blocks, 52 M) 51 / 43; Q8_0 4096 x
+// 4096 of 192 (50 M) 44 / 51, of 256 (67 M) 56 / 52.  Several matrices are one
+// launch here and as many (with a prologue, more) there: gate and up of 2 x
+// 14336 rows of 4096, 131 tokens (352 M) 101 / 130 us, 200 tokens (470 M)
+// 148 / 139.
 constexpr int kSmallMinTokens = 5;
-constexpr int kSmallMaxTokens = 64;
-bool use_small(uint32_t type, int nmat, const void *const *w, int m) {
-    static const int lo = tuning_knob("EXQ_SM_LO", kSmallMinTokens), hi = tuning_knob("EXQ_SM_HI", kSmallMaxTokens);
-    if (m < lo || m > hi) return false;
-    if (type == (uint32_t)kTypeQ8_0 || type == (uint32_t)kTypeQ6_K) return true;
-    if (type != (uint32_t)kTypeQ4_K) return false;
+bool use_small(uint32_t type, int nmat, const void *const *w, const int *n_out, int n_in, int m) {
+    static const int lo = tuning_knob("EXQ_SM_LO", kSmallMinTokens), hi = tuning_knob("EXQ_SM_HI", 0);
+    if (m < lo) return false;
+    if (type != (uint32_t)kTypeQ8_0 && type != (uint32_t)kTypeQ6_K && type != (uint32_t)kTypeQ4_K) return false;
+    const int blocks = (m + 63) / 64;
+    if (hi != 0 ? m > hi : blocks > 1) {
+        if (hi != 0) return false;
+        const double limit = type == (uint32_t)kTypeQ4_K ? 110e6 : type == (uint32_t)kTypeQ6_K ? 64e6 : 56e6;
+        if (type == (uint32_t)kTypeQ6_K && blocks > 5) return false;
+        double rows = 0.0;
+        for (int z = 0; z < nmat; ++z) rows += n_out[z];
+        if (rows * n_in * blocks > limit * (nmat == 1 ? 1.0 : 1.5 * nmat)) return false;
+    }
+    if (type != (uint32_t)kTypeQ4_K) return true;
     if (m >= gemm_min_tokens(type) && g.prefill_mode != EDGEXPU_HIP_PREFILL_EXACT_INT8) return false;
     for (int z = 0; z < nmat; ++z)
         if (!aligned16(w[z])) return false;
@@ -596,7 +613,7 @@ bool run_q8_product(uint32_t type, const void *w, int n_out, int n_in, int m, co
                     float *out, int ldo, hipStream_t st) {
     const size_t rb = edgexpu_hip_row_bytes(type, n_in);
     const size_t ab = act_bytes(type, n_in);
-    if (ldo == n_out && use_small(type, 1, &w, m))
+    if (ldo == n_out && use_small(type, 1, &w, &n_out, n_in, m))
         return run_small(type, 1, &w, &n_out, &bias, nullptr, &out, false, nullptr, nullptr, 0.0f, 0, xq, ab, m, n_in,
                          st);
     if (m >= gemm_min_tokens(type) && exact_gemm_type(type, 1, &w, &n_out, n_in, m)) {
@@ -641,7 +658,7 @@ bool run_linear_group(uint32_t type, int nmat, const void *const *w, const int *
                 return false;
         return true;
     }
-    if (use_small(type, nmat, w, m))
+    if (use_small(type, nmat, w, n_out, n_in, m))
         return run_small(type, nmat, w, n_out, bias, nullptr, out, false, x, nullptr, 0.0f, 0, nullptr, 0, m, n_in, st);
     // two to four tokens of the rows the streaming GEMV takes are quantized
     // inside its workgroups too; other long rows quantize once in their own
@@ -964,7 +981,7 @@ int edgexpu_hip_layer_linear_dev(int nmat, float *const *out, const float *x, co
                    ? 1
                    : 0;
     // a few tokens: the prologue in the pack, the residual in the product's store
-    if (use_small(type, nmat, w, m) && !outputs_overlap(nmat, out, residual, bias, n_out, m))
+    if (use_small(type, nmat, w, n_out, n_in, m) && !outputs_overlap(nmat, out, residual, bias, n_out, m))
         return run_small(type, nmat, w, n_out, bias, residual, out, false, x, pro == 1 ? norm_weight : x2, eps, pro,
                          nullptr, 0, m, n_in, st)
                    ? 1
@@ -1032,7 +1049,7 @@ int edgexpu_hip_gate_up_silu_dev(float *act, const float *x, const float *norm_w
                    : 0;
     }
     float *act_out[2] = {act, nullptr};
-    if (use_small(type, 2, wg, m) && !outputs_overlap(1, act_out, nullptr, bg, nn, m) &&
+    if (use_small(type, 2, wg, nn, n_in, m) && !outputs_overlap(1, act_out, nullptr, bg, nn, m) &&
         !outputs_overlap(1, act_out, nullptr, bg + 1, nn, m))
         return run_small(type, 2, wg, nn, bg, nullptr, act_out, true, x, norm_weight, eps, pro, nullptr, 0, m, n_in,
                          st)

@@ -1,4 +1,4 @@
-"""Products of 5 to 64 tokens (csrc/gemm_small.hip) against the oracle.
+"""Products of a few tokens, and of more against few rows (csrc/gemm_small.hip), against the oracle.
 
 Q4_K, Q6_K and Q8_0 rows on the integer matrix cores, 16 rows by up to 64
 tokens per workgroup with K split over its waves: every output within 1e-5 of
@@ -38,7 +38,7 @@ def scales(qt, w, xq):
 
 @pytest.mark.parametrize("qt,n_in", [(12, 256), (12, 2560), (12, 4352), (14, 256), (14, 2816), (14, 9728), (8, 32),
                                      (8, 576), (8, 2080)])
-@pytest.mark.parametrize("m", [5, 16, 17, 33, 64])
+@pytest.mark.parametrize("m", [5, 16, 17, 33, 64, 131])
 def test_small_vs_oracle(hipdev, ora, qt, n_in, m):
     """A group of ragged row counts (one below a tile, one past it, one row),
     with and without bias; equal to the call of each matrix alone and to the
