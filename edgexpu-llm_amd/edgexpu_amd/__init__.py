@@ -149,9 +149,14 @@ def _ptr(t) -> int | None:
 
 
 def _stream():
+    """The handle of torch's current stream on the current device, without the
+    Stream object torch.cuda.current_stream() builds on every call (2.9 us; the
+    handle alone 0.2 us, of the 10 to 14 us a layer call spends on the host)."""
     import torch
 
-    return torch.cuda.current_stream().cuda_stream
+    if not torch.cuda.is_initialized():  # the first call of the process sets the device up
+        return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 # ---------------------------------------------------------------- device API
