@@ -22,6 +22,12 @@ hipError_t launch_gemv_stream(int type, int nmat, const uint8_t *const *w, const
 
 using namespace exq;
 
+// gemv_q80_row.hip: one staged token of short Q8_0 rows
+bool gemv_q80_row_take(int type, int K, int m, long long rows, bool staged);
+hipError_t launch_gemv_q80_row(int nmat, const uint8_t *const *w, const int *n_out, const float *const *bias,
+                               const float *const *resid, float *const *out, int K, const float *x, const float *x2,
+                               const float *nw, float eps, int pro, bool pair, hipStream_t st);
+
 // Rows split over three waves (12-wave workgroups) are instantiated for one
 // staged token of Q4_K / Q6_K rows (knob EXQ_FUSED_KS3=0: never).
 static bool fused_with3(int type, int m, bool staged) {
@@ -299,6 +305,9 @@ hipError_t launch_gemv_fused_layer(int type, int nmat, const uint8_t *const *w, 
     // tokens of Q6_K rows of 9728; its rows equal this kernel's bit for bit
     long long rows = 0;
     for (int z = 0; z < nmat; ++z) rows += n_out[z];
+    // few Q8_0 rows, same words as below in a shorter launch
+    if (gemv_q80_row_take(type, K, m, rows, x != nullptr))
+        return launch_gemv_q80_row(nmat, w, n_out, bias, resid, out, K, x, x2, nw, eps, pro, pair, st);
     if (gemv_stream_take(type, K, m, rows, nmat, w, code, x != nullptr))
         return launch_gemv_stream(type, nmat, w, n_out, bias, resid, out, K, m, x, xq, x2, nw, eps, pro, pair, st);
     a.nblk = q8_0_family(type) ? K / kQK8_0 : K / kQKK;
