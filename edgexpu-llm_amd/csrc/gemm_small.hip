@@ -599,7 +599,11 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_small_kernel(SmallArgs a) {
         row[rt] = a.w[PAIR ? rt : z] + (size_t)min(row0 + (PAIR ? 0 : 16 * rt) + r16, n_out - 1) * a.row_bytes;
     constexpr int kGran = F::kType == kTypeQ8_0 ? 2 : 1;  // Q8_0 blocks go in pairs
     const int np = (a.nk + kGran - 1) / kGran;
-    const int k0 = kGran * (np * wave / nw), k1 = min(a.nk, kGran * (np * (wave + 1) / nw));
+    // in 64 bits: with 32-bit divisions the compiler schedules the Q4_K loops
+    // of three and four token tiles into 30 % more registers (down of 64
+    // tokens of 14336 x 4096 41 us, 31 us so)
+    const int k0 = kGran * (int)((long long)np * wave / nw);
+    const int k1 = min(a.nk, kGran * (int)((long long)np * (wave + 1) / nw));
 
     float acc[RT][TT][4];
 #pragma unroll

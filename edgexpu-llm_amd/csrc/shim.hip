@@ -440,12 +440,13 @@ bool use_exact_gemm(uint32_t type, int nmat, const void *const *w, const int *n_
 // again) stays below the line where the 128-token tiles of the prefill GEMMs
 // catch up.  Measured, few-token / prefill, one matrix: Q4_K 4096 x 4096 of
 // 512 tokens (134 M) 48 / 53 us, 4096 x 14336 of 128 (117 M) 50 / 49, 2560 x
-// 9728 of 256 (100 M) 52 / 48; Q6_K 9728 x 2560 of 128 (50 M) 49 / 52, of 256
-// (100 M) 70 / 62, 2560 x 2560 of 512 (8 blocks, 52 M) 51 / 43; Q8_0 4096 x
-// 4096 of 192 (50 M) 44 / 51, of 256 (67 M) 56 / 52.  Several matrices are one
-// launch here and as many (with a prologue, more) there: gate and up of 2 x
-// 14336 rows of 4096, 131 tokens (352 M) 101 / 130 us, 200 tokens (470 M)
-// 148 / 139.
+// 9728 of 256 (100 M) 52 / 48; rows of 8192 and more, whose few tiles the
+// prefill GEMM splits four ways at most: 14336 x 4096 of 192 (176 M) 62 / 84;
+// Q6_K 9728 x 2560 of 192 (75 M) 50 / 60, of 256 (100 M) 70 / 62, 2560 x 2560
+// of 512 (8 blocks, 52 M) 51 / 43; Q8_0 4096 x 4096 of 192 (50 M) 44 / 51, of
+// 256 (67 M) 56 / 52.  Several matrices are one launch here and as many (with
+// a prologue, more) there: gate and up of 2 x 14336 rows of 4096, 131 tokens
+// (352 M) 102 / 119 us, 200 tokens (470 M) 148 / 132.
 constexpr int kSmallMinTokens = 5;
 bool use_small(uint32_t type, int nmat, const void *const *w, const int *n_out, int n_in, int m) {
     static const int lo = tuning_knob("EXQ_SM_LO", kSmallMinTokens), hi = tuning_knob("EXQ_SM_HI", 0);
@@ -454,11 +455,13 @@ bool use_small(uint32_t type, int nmat, const void *const *w, const int *n_out, 
     const int blocks = (m + 63) / 64;
     if (hi != 0 ? m > hi : blocks > 1) {
         if (hi != 0) return false;
-        const double limit = type == (uint32_t)kTypeQ4_K ? 110e6 : type == (uint32_t)kTypeQ6_K ? 64e6 : 56e6;
+        const double limit = type == (uint32_t)kTypeQ4_K   ? (n_in >= 8192 ? 220e6 : 110e6)
+                             : type == (uint32_t)kTypeQ6_K ? 80e6
+                                                           : 56e6;
         if (type == (uint32_t)kTypeQ6_K && blocks > 5) return false;
         double rows = 0.0;
         for (int z = 0; z < nmat; ++z) rows += n_out[z];
-        if (rows * n_in * blocks > limit * (nmat == 1 ? 1.0 : 1.5 * nmat)) return false;
+        if (rows * n_in * blocks > limit * (nmat == 1 ? 1.0 : 1.75 * nmat)) return false;
     }
     if (type != (uint32_t)kTypeQ4_K) return true;
     if (m >= gemm_min_tokens(type) && g.prefill_mode != EDGEXPU_HIP_PREFILL_EXACT_INT8) return false;
