@@ -25,24 +25,59 @@
 
 namespace exq {
 
-// One workgroup of 256 threads per row of n elements.
+// One workgroup of 256 threads per row of n elements.  vec: rows of whole,
+// aligned float4s, up to 4096 elements of which stay in registers between the
+// two passes, their loads issued together (a launch is one chain of latencies:
+// in front of the q/k/v of four tokens of 4096, 14.6 us for the call element
+// by element, 12.1 us so).
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                      float *__restrict__ out, int n, float eps) {
+                                                      float *__restrict__ out, int n, float eps, int vec) {
     __shared__ double part[4];
     const size_t row = blockIdx.x;
     const float *xr = x + row * (size_t)n;
     float *orow = out + row * (size_t)n;
+    const int tid = threadIdx.x, n4 = n >> 2;
+    constexpr int kKeep = 4;
+    float4 xv[kKeep], wv[kKeep];
+    const auto square = [](const float4 v) {  // a float square is exact in double
+        return ((double)v.x * (double)v.x + (double)v.y * (double)v.y) +
+               ((double)v.z * (double)v.z + (double)v.w * (double)v.w);
+    };
     double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) {
-        const double v = (double)xr[i];
-        s += v * v;  // a float square is exact in double
+    if (vec) {
+        const float4 *x4 = reinterpret_cast<const float4 *>(xr), *w4 = reinterpret_cast<const float4 *>(w);
+#pragma unroll
+        for (int k = 0; k < kKeep; ++k) xv[k] = x4[min(tid + 256 * k, n4 - 1)];
+#pragma unroll
+        for (int k = 0; k < kKeep; ++k) wv[k] = w4[min(tid + 256 * k, n4 - 1)];
+#pragma unroll
+        for (int k = 0; k < kKeep; ++k) s += tid + 256 * k < n4 ? square(xv[k]) : 0.0;
+        for (int i = tid + 256 * kKeep; i < n4; i += 256) s += square(x4[i]);
+    } else {
+        for (int i = tid; i < n; i += 256) {
+            const double v = (double)xr[i];
+            s += v * v;
+        }
     }
     s = wave_sum_f64(s);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    if ((tid & 63) == 0) part[tid >> 6] = s;
     __syncthreads();
     const double ss = (part[0] + part[1]) + (part[2] + part[3]);
     const float scale = rms_scale(ss, n, eps);
-    for (int i = threadIdx.x; i < n; i += 256) {
+    if (vec) {
+        float4 *o4 = reinterpret_cast<float4 *>(orow);
+        const auto norm = [scale](const float4 v, const float4 g) {
+            const float a = v.x * scale, b = v.y * scale, c = v.z * scale, d = v.w * scale;
+            return make_float4(a * g.x, b * g.y, c * g.z, d * g.w);
+        };
+#pragma unroll
+        for (int k = 0; k < kKeep; ++k)
+            if (tid + 256 * k < n4) o4[tid + 256 * k] = norm(xv[k], wv[k]);
+        for (int i = tid + 256 * kKeep; i < n4; i += 256)
+            o4[i] = norm(reinterpret_cast<const float4 *>(xr)[i], reinterpret_cast<const float4 *>(w)[i]);
+        return;
+    }
+    for (int i = tid; i < n; i += 256) {
         const float v = xr[i] * scale;
         orow[i] = v * w[i];
     }
@@ -67,7 +102,8 @@ __global__ __launch_bounds__(256) void elementwise_kernel(const float *__restric
 using namespace exq;
 
 hipError_t launch_rmsnorm(const float *x, const float *w, float *out, int m, int n, float eps, hipStream_t st) {
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)m), dim3(256), 0, st, x, w, out, n, eps);
+    const int vec = n % 4 == 0 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15u) == 0;
+    hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)m), dim3(256), 0, st, x, w, out, n, eps, vec);
     return hipGetLastError();
 }
 
