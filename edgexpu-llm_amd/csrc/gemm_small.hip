@@ -745,7 +745,7 @@ static hipError_t small_dispatch(const SmallArgs &a, int rt, int tt, bool pair, 
 #define SM_CASE(T)                                                      \
     case T:                                                             \
         if (pair)                                                       \
-            small_launch<F, (2), T, true>(a, tiles, nw, st); \
+            small_launch<F, 2, T, true>(a, tiles, nw, st);              \
         else if (rt == 2)                                               \
             small_launch<F, 2, T, false>(a, tiles, nw, st);             \
         else                                                            \

@@ -454,7 +454,7 @@ bool use_small(uint32_t type, int nmat, const void *const *w, const int *n_out, 
     if (type != (uint32_t)kTypeQ8_0 && type != (uint32_t)kTypeQ6_K && type != (uint32_t)kTypeQ4_K) return false;
     const int blocks = (m + 63) / 64;
     if (hi != 0 ? m > hi : blocks > 1) {
-        if (hi != 0) return false;
+        if (hi != 0 || blocks > 4096) return false;  // (token blocks are a launch's y dimension)
         const double limit = type == (uint32_t)kTypeQ4_K   ? (n_in >= 8192 ? 220e6 : 110e6)
                              : type == (uint32_t)kTypeQ6_K ? 80e6
                                                            : 56e6;
