@@ -135,7 +135,7 @@ int edgexpu_hip_weight_n_in(const edgexpu_hip_weight *w);
  * bytes) must start at an even one: an odd one is refused with error -2.
  * GGUF tensors in a device copy of a file's data section always qualify.
  * Blocks at 16-byte addresses can take the streaming GEMV and logits (Q4_K,
- * Q6_K) and the matrix-core prefill (Q4_K; the others need even addresses);
+ * Q6_K) and the matrix-core products (Q4_K; the others need even addresses);
  * blocks elsewhere take the fused GEMV, with the same results. ---- */
 
 /* out[t*n_out + o] = bias[o] + dot(W[o], q8(x[t]))  for t < m.
