@@ -296,7 +296,8 @@ hipError_t launch_gemv_fused_layer(int type, int nmat, const uint8_t *const *w, 
     bool any_resid = false;
     for (int z = 0; z < nmat; ++z) any_resid = any_resid || a.resid[z] != nullptr;
     const int code = pro | (any_resid ? 4 : 0) | (pair ? 8 : 0);
-    if (code != 0 && (x == nullptr || m != 1 || code == 5 || (pair && pro == 2) || (pro == 1 && nw == nullptr) ||
+    // (a residual alone: several tokens too, on the streaming kernel below)
+    if (code != 0 && (x == nullptr || (m != 1 && code != 4) || code == 5 || (pair && pro == 2) || (pro == 1 && nw == nullptr) ||
                       (pro == 2 && x2 == nullptr)))
         return hipErrorInvalidValue;
     // Q4_K rows at the decode lengths: the streaming kernel (one token: every

@@ -349,7 +349,7 @@ struct StreamGeom {
     static_assert(!(FL & kSRow3) || (Q6 && F32 && M == 1), "row triples: one token of Q6_K f32 logits");
     static_assert(!(FL & kSArgmax) || (F32 && M == 1), "argmax keys: one f32 token");
     static_assert(AREA % 16 == 0, "slot alignment");
-    static_assert(M == 1 || (FL & ~(kSF32 | kSRow2)) == 0, "several tokens: plain projections");
+    static_assert(M == 1 || (FL & ~(kSF32 | kSRow2 | kSRes)) == 0, "several tokens: projections, plain or with a residual");
     static_assert(XREG || (FL & kSXq) == 0, "Q8_K block input: the slices in registers");
     static_assert(!(FL & kSRow2) || ((FL & ~(kSRow2 | 1)) == 0 && !Q6),
                   "row pairs: Q4_K projections, RMSNorm prologue (one token) or none");
@@ -669,7 +669,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_q4k(StreamArgs a) {
                 e.b0 = bias != nullptr ? bias[row] : 0.0f;
             }
             if constexpr (kPair) e.b1 = a.bias[1] != nullptr ? a.bias[1][row] : 0.0f;
-            if constexpr (kRes) e.r = resid != nullptr ? resid[row] : 0.0f;
+            if constexpr (kRes && M == 1) e.r = resid != nullptr ? resid[row] : 0.0f;
         }
         return e;
     };
@@ -686,12 +686,18 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_q4k(StreamArgs a) {
         const float *bias, *resid;
         lane_out(step < last ? step : 0, out, row, bias, resid, n_out);
         if (lane < n && step < last) {
-            // out = resid + (bias + dot) (src/native.c:2571-2580); pairs: silu(gate) * up
+            // out = resid + (bias + dot) (src/native.c:2571-2580); pairs: silu(gate) * up.
+            // Several tokens' residuals are read here, together (kept from the
+            // start they would cost a register a token through the loop)
+            float res[M];
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                res[m] = !kRes ? 0.0f : M == 1 ? e.r : resid != nullptr ? resid[(size_t)m * n_out + row] : 0.0f;
 #pragma unroll
             for (int m = 0; m < M; ++m) {
                 const float v = e.b0 + keep[m];
                 float o = v;
-                if constexpr (kRes) o = resid != nullptr ? e.r + v : v;
+                if constexpr (kRes) o = resid != nullptr ? res[m] + v : v;
                 if constexpr (kPair) o = silu_f32(v) * (e.b1 + keep1[m]);
                 if constexpr (kRow2) {
                     out[(size_t)m * n_out + 2 * row] = o;
@@ -1000,9 +1006,9 @@ hipError_t launch_stream_tokens(int m, const StreamArgs &a, hipStream_t st) {
         const long long per_gen = (long long)device_cus() * 8;
         if (((long long)a.nrows + per_gen - 1) / per_gen <= 3) {
             switch (m) {
-                case 2: return launch_stream_geom<KSB, 8, 1, 0, false, 2, TYPE>(a, st);
-                case 3: return launch_stream_geom<KSB, 8, 1, 0, false, 3, TYPE>(a, st);
-                case 4: return launch_stream_geom<KSB, 8, 1, 0, false, 4, TYPE>(a, st);
+                case 2: return launch_stream_geom<KSB, 8, 1, FL, false, 2, TYPE>(a, st);
+                case 3: return launch_stream_geom<KSB, 8, 1, FL, false, 3, TYPE>(a, st);
+                case 4: return launch_stream_geom<KSB, 8, 1, FL, false, 4, TYPE>(a, st);
                 default: return hipErrorInvalidValue;
             }
         }
@@ -1047,15 +1053,16 @@ int gemv_stream_mode() { return g_gemv_mode; }
 // True when the streaming GEMV can take (type, K, m).
 // code: prologue (bits 0-1), residual (4), gate/up pairs (8); staged: f32
 // tokens (not Q8_K block bytes).  Q4_K: one token of rows of 2560, 4096 or
-// 14336, or plain projections of m = 2..4 staged tokens of those rows.
-// Q6_K: staged tokens of rows of 9728 (the hybrid ~4B down projection), one
-// (any variant but pairs) or two to four (plain projections).
+// 14336, or projections of m = 2..4 staged tokens of those rows, plain or with
+// a residual.  Q6_K: staged tokens of rows of 9728 (the hybrid ~4B down
+// projection), one (any variant but pairs) or two to four (plain or with a
+// residual: the add was a launch of 2.4-4 us of its own).
 bool gemv_stream_supported(int type, int K, int m, int code, bool staged) {
     if (type == kTypeQ4_K) {
         if (m == 1) return K == 2560 || K == 4096 || K == 14336;
-        return m >= 2 && m <= 4 && staged && code == 0 && (K == 2560 || K == 4096 || K == 14336);
+        return m >= 2 && m <= 4 && staged && (code == 0 || code == kSRes) && (K == 2560 || K == 4096 || K == 14336);
     }
-    if (type == kTypeQ6_K) return K == 9728 && staged && (m == 1 ? (code & 8) == 0 : m <= 4 && code == 0);
+    if (type == kTypeQ6_K) return K == 9728 && staged && (m == 1 ? (code & 8) == 0 : m <= 4 && (code == 0 || code == kSRes));
     return false;
 }
 
@@ -1157,7 +1164,16 @@ hipError_t launch_gemv_stream(int type, int nmat, const uint8_t *const *w, const
     // [2560 x 9728]: 10.2 us; a deep start 11.6, two slots 11.9, 12 waves
     // per CU 10.2 but 13.2 at 4096 rows)
     if (type == kTypeQ6_K)
-        return m > 1 ? launch_stream_tokens<38, 1, kTypeQ6_K>(m, a, st) : launch_stream_q6k<38, 8, 1>(fl, a, st);
+        return m == 1    ? launch_stream_q6k<38, 8, 1>(fl, a, st)
+               : any_res ? launch_stream_tokens<38, 1, kTypeQ6_K, kSRes>(m, a, st)
+                         : launch_stream_tokens<38, 1, kTypeQ6_K>(m, a, st);
+    if (m > 1 && any_res) {
+        switch (K) {
+            case 2560: return launch_stream_tokens<10, 2, kTypeQ4_K, kSRes>(m, a, st);
+            case 4096: return launch_stream_tokens<16, 2, kTypeQ4_K, kSRes>(m, a, st);
+            default: return launch_stream_tokens<56, 1, kTypeQ4_K, kSRes>(m, a, st);
+        }
+    }
     if (m > 1) {
         switch (K) {
             case 2560:

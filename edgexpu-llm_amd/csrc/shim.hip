@@ -989,6 +989,17 @@ int edgexpu_hip_layer_linear_dev(int nmat, float *const *out, const float *x, co
                          nullptr, 0, m, n_in, st)
                    ? 1
                    : 0;
+    // two to four tokens of the streaming GEMV's rows: the residual in its store
+    long long rows = 0;
+    for (int z = 0; z < nmat; ++z) rows += n_out[z];
+    if (pro == 0 && any_resid && m > 1 && m <= kFusedMaxTokens &&
+        gemv_stream_take((int)type, n_in, m, rows, nmat, (const uint8_t *const *)w, 4, true) &&
+        !outputs_overlap(nmat, out, residual, bias, n_out, m))
+        return hip_ok(launch_gemv_fused_layer((int)type, nmat, (const uint8_t *const *)w, n_out, bias, residual, out,
+                                              rb, n_in, m, x, nullptr, nullptr, eps, 0, nullptr, 0, st),
+                      "layer_linear stream")
+                   ? 1
+                   : 0;
     // otherwise the same arithmetic in steps: prologue kernel, projection,
     // residual add (the projection writes to the workspace first, so out may
     // be the residual)

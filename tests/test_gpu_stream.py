@@ -364,6 +364,36 @@ def test_q6k_layer_variants_fused_equals_stream(hipdev, ora, pro):
     assert np.array_equal(bits(f[0]), bits(s[0]))
 
 
+@pytest.mark.parametrize("qt,n_in,n_outs", [(12, 2560, (77,)), (12, 4096, (2560, 33)), (12, 4096, (30000,)),
+                                            (12, 14336, (2050,)), (14, 9728, (2560,))])
+@pytest.mark.parametrize("m", [2, 3, 4])
+def test_tokens_residual_in_the_store(hipdev, qt, n_in, n_outs, m):
+    """Two to four tokens with a residual (also over itself) in the streaming
+    kernel's store equal the projection followed by the add, word for word; a
+    matrix without one, and an output that is another matrix's residual (which
+    takes the steps), too."""
+    rng = np.random.default_rng(n_in + m + sum(n_outs))
+    ws = [dev(synth.np_weights(qt, n, n_in, rng)) for n in n_outs]
+    x = dev(synth.np_activations(m, n_in, rng))
+    bs = [dev(rng.normal(0, 0.3, n).astype(np.float32)) for n in n_outs]
+    res = [dev(rng.normal(0, 4, (m, n)).astype(np.float32)) for n in n_outs]
+    plain = E.linear_quant_group(ws, qt, x, list(n_outs), n_in, biases=bs)
+    want = [bits(E.add(r, p).cpu().numpy()) for r, p in zip(res, plain)]
+    into = [r.clone() for r in res]
+    E.layer_linear(ws, qt, x, list(n_outs), n_in, biases=bs, residuals=into, outs=into)
+    for z in range(len(n_outs)):
+        assert np.array_equal(bits(into[z].cpu().numpy()), want[z]), f"matrix {z}"
+    if len(n_outs) > 1:
+        got = E.layer_linear(ws, qt, x, list(n_outs), n_in, biases=bs, residuals=[res[0], None])
+        assert np.array_equal(bits(got[0].cpu().numpy()), want[0])
+        assert np.array_equal(bits(got[1].cpu().numpy()), bits(plain[1].cpu().numpy()))
+    o0 = res[0].clone()
+    got = E.layer_linear([ws[0], ws[0]], qt, x, [n_outs[0]] * 2, n_in, biases=[bs[0]] * 2, residuals=[res[0], o0],
+                         outs=[o0, torch.empty_like(o0)])
+    assert np.array_equal(bits(got[0].cpu().numpy()), want[0])
+    assert np.array_equal(bits(got[1].cpu().numpy()), bits(E.add(o0, plain[0]).cpu().numpy()))
+
+
 def test_gemv_mode_switch(hipdev):
     L = hipdev
     assert L.gemv_mode() == AUTO
