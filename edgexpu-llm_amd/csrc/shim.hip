@@ -117,6 +117,18 @@ constexpr int kStageMaxK = 4096;
 // ... except one token's Q8_K activation up to this many elements, which
 // the 16-wave workgroups of the row-split GEMV quantize in one round.
 constexpr int kStageMaxKWide = 16384;
+// A workspace that grows by doubling from 4 MiB (the few-token pack of 200
+// tokens of 14336 elements) and keeps the buffers it outgrew until shutdown, so
+// that a captured graph's pointers stay good; together they are smaller than
+// the current one.
+struct KeptWs {
+    static constexpr size_t kFirst = (size_t)4 << 20;
+    static constexpr int kMaxOld = 40;
+    void *p = nullptr;
+    size_t cap = 0;
+    void *old[kMaxOld] = {};
+    int n_old = 0;
+};
 constexpr int kArgmaxParts = 4096;  // per token: the two-pass argmax's 1024, or one key per wave of a logits launch
 
 struct State {
@@ -133,8 +145,7 @@ struct State {
     void *lws = nullptr;    // layer entry: prologue activation and pre-residual outputs
     size_t lws_cap = 0;
     int prefill_mode = 0;   // EDGEXPU_HIP_PREFILL_EXACT_INT8 / _F16
-    void *tws = nullptr;    // few-token GEMM: activation pack
-    size_t tws_cap = 0;
+    KeptWs tws;             // few-token GEMM: activation pack
     void *gws = nullptr;    // exact prefill GEMM: activation pack
     size_t gws_cap = 0;
     size_t dbuf_cap = 0;
@@ -336,21 +347,30 @@ void *gemm_ws(size_t bytes) {
     return g.gws;
 }
 
-// Workspace of the few-token GEMM (the activation pack), grown on demand in
-// steps of 4 MiB (the pack of 200 tokens of 14336 elements), so that a step
-// captured in a graph keeps its address whatever sizes run beside it.
+// Workspace of the few-token GEMM (the activation pack).  Calls of very
+// different sizes take it (an 8-token step, a q/k/v group of 1408 tokens), so
+// it must be able to grow under a step captured in a graph.
 void *small_ws(size_t bytes) {
-    if (bytes <= g.tws_cap) return g.tws;
-    if (g.tws != nullptr) {
-        if (!hip_ok(hipDeviceSynchronize(), "few-token workspace sync")) return nullptr;
-        (void)hipFree(g.tws);
-        g.tws = nullptr;
-        g.tws_cap = 0;
+    KeptWs &k = g.tws;
+    if (bytes <= k.cap) return k.p;
+    size_t cap = KeptWs::kFirst;
+    while (cap < bytes) cap *= 2;
+    if (k.n_old == KeptWs::kMaxOld) {  // (not reached: every growth doubles)
+        set_error(-5, "few-token workspace: too many growths");
+        return nullptr;
     }
-    const size_t cap = align_up(bytes, (size_t)4 << 20);
-    if (!hip_ok(hipMalloc(&g.tws, cap), "hipMalloc few-token workspace")) return nullptr;
-    g.tws_cap = cap;
-    return g.tws;
+    void *p = nullptr;
+    if (!hip_ok(hipMalloc(&p, cap), "hipMalloc few-token workspace")) return nullptr;
+    if (k.p != nullptr) k.old[k.n_old++] = k.p;
+    k.p = p;
+    k.cap = cap;
+    return p;
+}
+
+void free_kept(KeptWs &k) {
+    for (int i = 0; i < k.n_old; ++i) (void)hipFree(k.old[i]);
+    if (k.p != nullptr) (void)hipFree(k.p);
+    k = KeptWs();
 }
 
 // Formats with an exact matrix-core prefill GEMM: Q4_K straight from its
@@ -742,7 +762,7 @@ void edgexpu_hip_shutdown(void) {
     if (g.sws) (void)hipFree(g.sws);
     if (g.lws) (void)hipFree(g.lws);
     if (g.gws) (void)hipFree(g.gws);
-    if (g.tws) (void)hipFree(g.tws);
+    free_kept(g.tws);
     (void)hipStreamDestroy(g.stream);
     const int err = g.err;
     char msg[sizeof(g.msg)];
