@@ -109,7 +109,8 @@ constexpr int kFusedMaxTokens = 4;
 // 40 / 41 / 46 us at 16 / 32 / 64 ([4096 x 4096]: GEMV 18 / 31 / 55, GEMM
 // 29 / 31 / 35).  Q5_K pays a weight repack per call: GEMV 31 / 55 us at 16 /
 // 32 tokens against 47 / 48, so it switches at 32.
-int gemm_min_tokens(uint32_t type) { return type == (uint32_t)kTypeQ5_K ? 32 : 16; }
+constexpr int kPrefillTokens = 16;
+int gemm_min_tokens(uint32_t type) { return type == (uint32_t)kTypeQ5_K ? 32 : kPrefillTokens; }
 // Rows up to this many elements quantize the activation inside the GEMV
 // workgroups; longer rows quantize it once in its own launch (the in-kernel
 // staging costs one load latency per 8192 elements per workgroup) ...
@@ -145,7 +146,7 @@ struct State {
     void *lws = nullptr;    // layer entry: prologue activation and pre-residual outputs
     size_t lws_cap = 0;
     int prefill_mode = 0;   // EDGEXPU_HIP_PREFILL_EXACT_INT8 / _F16
-    KeptWs tws;             // few-token GEMM: activation pack
+    KeptWs tws[2];          // few-token GEMM: activation pack of decode, of prefill token counts
     void *gws = nullptr;    // exact prefill GEMM: activation pack
     size_t gws_cap = 0;
     size_t dbuf_cap = 0;
@@ -349,9 +350,11 @@ void *gemm_ws(size_t bytes) {
 
 // Workspace of the few-token GEMM (the activation pack).  Calls of very
 // different sizes take it (an 8-token step, a q/k/v group of 1408 tokens), so
-// it must be able to grow under a step captured in a graph.
-void *small_ws(size_t bytes) {
-    KeptWs &k = g.tws;
+// it must be able to grow under a step captured in a graph.  Below 16 tokens
+// it is another buffer than from 16, as the GEMVs' and the prefill GEMMs'
+// workspaces are: a decode step and a prefill on two streams share none.
+void *small_ws(int m, size_t bytes) {
+    KeptWs &k = g.tws[m < kPrefillTokens ? 0 : 1];
     if (bytes <= k.cap) return k.p;
     size_t cap = KeptWs::kFirst;
     while (cap < bytes) cap *= 2;
@@ -496,7 +499,7 @@ bool use_small(uint32_t type, int nmat, const void *const *w, const int *n_out, 
 bool run_small(uint32_t type, int nmat, const void *const *w, const int *n_out, const float *const *bias,
                const float *const *resid, float *const *out, bool pair, const float *x, const float *y, float eps,
                int pro, const uint8_t *xq, size_t xq_stride, int m, int n_in, hipStream_t st) {
-    uint8_t *pack = (uint8_t *)small_ws(gemm_small_pack_bytes((int)type, m, n_in));
+    uint8_t *pack = (uint8_t *)small_ws(m, gemm_small_pack_bytes((int)type, m, n_in));
     if (pack == nullptr) return false;
     const hipError_t e = x != nullptr ? launch_small_pack((int)type, x, y, eps, pro, m, n_in, pack, st)
                                       : launch_small_pack_blocks((int)type, xq, xq_stride, m, n_in, pack, st);
@@ -762,7 +765,7 @@ void edgexpu_hip_shutdown(void) {
     if (g.sws) (void)hipFree(g.sws);
     if (g.lws) (void)hipFree(g.lws);
     if (g.gws) (void)hipFree(g.gws);
-    free_kept(g.tws);
+    for (KeptWs &k : g.tws) free_kept(k);
     (void)hipStreamDestroy(g.stream);
     const int err = g.err;
     char msg[sizeof(g.msg)];

@@ -62,3 +62,28 @@ def test_captured_call_survives_larger_calls(fresh, m):
                 assert np.array_equal(bits(o), bits(r)), (big_m, big_k, rep, z)
             assert np.array_equal(bits(again), bits(first)), (big_m, big_k, rep)
         assert all(bool(torch.isnan(j).all()) for j in junk), "a replay wrote into another tensor"
+
+
+@pytest.mark.parametrize("qt", [8, 12, 14])
+def test_decode_and_prefill_on_two_streams(fresh, qt):
+    """A few-token call of a decode step beside one of a prefill, each on its
+    own stream: the two packs are in different buffers, so every result is
+    that of the call alone."""
+    rng = np.random.default_rng(qt)
+    n_out, n_in = 48, 4096
+    w = dev(synth.np_weights(qt, n_out, n_in, rng))
+    xs = [dev(synth.np_activations(m, n_in, rng)) for m in (8, 15, 700)]
+    want = [E.linear_quant_batch(w, qt, x, n_out, n_in).clone() for x in xs]
+    torch.cuda.synchronize()
+    decode, prefill = torch.cuda.Stream(), torch.cuda.Stream()
+    got = [[torch.empty_like(o) for _ in range(40)] for o in want]
+    for i in range(40):
+        with torch.cuda.stream(prefill):
+            E.linear_quant_batch(w, qt, xs[2], n_out, n_in, out=got[2][i])
+        with torch.cuda.stream(decode):
+            for z in (0, 1):
+                E.linear_quant_batch(w, qt, xs[z], n_out, n_in, out=got[z][i])
+    torch.cuda.synchronize()
+    for z, o in enumerate(want):
+        for i in range(40):
+            assert np.array_equal(bits(got[z][i]), bits(o)), (z, i)
