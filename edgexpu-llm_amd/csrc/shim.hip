@@ -362,8 +362,14 @@ void *small_ws(int m, size_t bytes) {
         set_error(-5, "few-token workspace: too many growths");
         return nullptr;
     }
+    // (allocating is no stream work: allowed while some stream is captured, as
+    // for a call that is captured before any eager one of its size)
     void *p = nullptr;
-    if (!hip_ok(hipMalloc(&p, cap), "hipMalloc few-token workspace")) return nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (!hip_ok(hipThreadExchangeStreamCaptureMode(&mode), "capture mode")) return nullptr;
+    const hipError_t e = hipMalloc(&p, cap);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!hip_ok(e, "hipMalloc few-token workspace")) return nullptr;
     if (k.p != nullptr) k.old[k.n_old++] = k.p;
     k.p = p;
     k.cap = cap;

@@ -87,3 +87,25 @@ def test_decode_and_prefill_on_two_streams(fresh, qt):
     for z, o in enumerate(want):
         for i in range(40):
             assert np.array_equal(bits(got[z][i]), bits(o)), (z, i)
+
+
+@pytest.mark.parametrize("m", [8, 40])
+def test_capture_before_any_few_token_call(fresh, m):
+    """Captured with the other paths' workspaces in place but no earlier call
+    of a few tokens: the capture succeeds, and every replay is the eager result."""
+    rng = np.random.default_rng(m)
+    n_out, n_in = 48, 4096
+    w = dev(synth.np_weights(12, n_out, n_in, rng))
+    x = dev(synth.np_activations(m, n_in, rng))
+    E.logits(w, 12, x[:1].contiguous(), n_out, n_in)
+    out = torch.empty((m, n_out), device="cuda:0")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):  # global capture mode
+        E.linear_quant_batch(w, 12, x, n_out, n_in, out=out)
+    want = E.linear_quant_batch(w, 12, x, n_out, n_in)
+    for rep in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(out), bits(want)), rep
