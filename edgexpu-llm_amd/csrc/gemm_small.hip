@@ -789,7 +789,13 @@ hipError_t launch_gemm_small(int type, int nmat, const uint8_t *const *w, const 
     long long rows = 0;
     for (int z = 0; z < nmat; ++z) rows += n_out[z];
     static const int k_rt = tuning_knob("EXQ_SM_RT", 0);
-    const int rt = pair ? 2 : k_rt ? k_rt : (rows >= 16 * 512 ? 2 : 1);
+    // two row tiles a wave where there are workgroups enough: the operands are
+    // loaded once for both.  Q6_K from the second token tile keeps one: twice
+    // the operands and accumulators leave half the waves per CU (9728 rows of
+    // 2560: 20 tokens 26.5 us with two, 21.9 with one; 64 tokens 46.8 and 30.5;
+    // 16 tokens of 8192 rows 12.1 and 13.0)
+    const bool wide = rows >= 16 * 512 && (type != kTypeQ6_K || tt == 1);
+    const int rt = pair ? 2 : k_rt ? k_rt : wide ? 2 : 1;
     int tiles = 0;
     for (int z = 0; z < nmat; ++z) {
         a.w[z] = w[z];

@@ -38,11 +38,12 @@ def scales(qt, w, xq):
 
 @pytest.mark.parametrize("qt,n_in", [(12, 256), (12, 2560), (12, 4352), (14, 256), (14, 2816), (14, 9728), (8, 32),
                                      (8, 576), (8, 2080)])
-@pytest.mark.parametrize("m", [5, 16, 17, 33, 64, 131])
+@pytest.mark.parametrize("m", [5, 16, 17, 33, 64, 70, 100, 131])
 def test_small_vs_oracle(hipdev, ora, qt, n_in, m):
     """A group of ragged row counts (one below a tile, one past it, one row),
     with and without bias; equal to the call of each matrix alone and to the
-    call over quantized blocks bit for bit."""
+    call over quantized blocks bit for bit.  70 and 100 tokens are five and
+    seven token tiles in two blocks, whose last one reads past the pack's."""
     n_outs = (15, 33, 1)
     rng = np.random.default_rng(100 * qt + n_in + m)
     ws = [synth.np_weights(qt, n, n_in, rng) for n in n_outs]
@@ -61,6 +62,21 @@ def test_small_vs_oracle(hipdev, ora, qt, n_in, m):
         assert np.array_equal(bits(got), bits(one)), f"matrix {z} alone"
         blk = E.gemv_q8(wd[z], qt, dev(xq), m, n, n_in, bias=bd[z]).cpu().numpy()
         assert np.array_equal(bits(got), bits(blk)), f"matrix {z} from blocks"
+
+
+@pytest.mark.parametrize("qt,n_in", [(12, 256), (14, 512), (8, 96)])
+@pytest.mark.parametrize("m", [12, 16, 17, 70, 100])
+def test_small_many_rows(hipdev, qt, n_in, m):
+    """From 8192 rows a wave may take two row tiles: the same words as the rows
+    computed in parts below that, the last tiles ragged."""
+    n_out = 8203
+    rng = np.random.default_rng(qt + m)
+    w = dev(synth.np_weights(qt, n_out, n_in, rng))
+    x = dev(synth.np_activations(m, n_in, rng))
+    got = E.linear_quant_batch(w, qt, x, n_out, n_in).cpu().numpy()
+    for r0, r1 in ((0, 3000), (3000, 8170), (8170, n_out)):
+        part = E.linear_quant_batch(w[r0:r1].contiguous(), qt, x, r1 - r0, n_in).cpu().numpy()
+        assert np.array_equal(bits(got[:, r0:r1]), bits(part)), r0
 
 
 @pytest.mark.parametrize("qt,n_in,n_out", [(12, 4096, 8200), (14, 2560, 300), (8, 576, 100)])
