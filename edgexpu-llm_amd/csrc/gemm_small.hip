@@ -686,6 +686,29 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_small_kernel(SmallArgs a) {
 
 using namespace exq;
 
+// True when a matrix of n_out rows of K elements takes this GEMM at m tokens:
+// Q4_K, Q6_K and Q8_0 from kSmallMinTokens tokens, up to 64 always, beyond that
+// while rows x K x (64-token blocks, each of which reads the weights again)
+// stays below the line where the 128-token tiles of the prefill GEMMs catch
+// up.  Measured, few-token / prefill: Q4_K 4096 x 4096 of 512 tokens (134 M)
+// 48 / 53 us, 14336 rows of 4096 at 128 (117 M) 50 / 49, 9728 of 2560 at 256
+// (100 M) 52 / 48; rows of 8192 and more, whose few tiles the prefill GEMM
+// splits four ways at most: 4096 rows of 14336 at 192 (176 M) 62 / 84; Q6_K
+// 2560 rows of 9728 at 192 (75 M) 50 / 60, at 256 (100 M) 70 / 62, 2560 of 2560
+// at 512 (8 blocks, 52 M) 51 / 43; Q8_0 4096 x 4096 of 192 (50 M) 44 / 51, of
+// 256 (67 M) 56 / 52.
+constexpr int kSmallMinTokens = 5;
+bool gemm_small_take(int type, int n_out, int K, int m) {
+    static const int lo = tuning_knob("EXQ_SM_LO", kSmallMinTokens), hi = tuning_knob("EXQ_SM_HI", 0);
+    if ((type != kTypeQ8_0 && type != kTypeQ6_K && type != kTypeQ4_K) || m < lo) return false;
+    const int blocks = (m + 63) / 64;
+    if (hi != 0) return m <= hi;
+    if (blocks == 1) return true;
+    if (blocks > 4096 || (type == kTypeQ6_K && blocks > 5)) return false;  // (token blocks are a launch's y dimension)
+    const double limit = type == kTypeQ4_K ? (K >= 8192 ? 220e6 : 110e6) : type == kTypeQ6_K ? 80e6 : 56e6;
+    return (double)n_out * K * blocks <= limit;
+}
+
 size_t gemm_small_pack_bytes(int type, int m, int K) {
     const size_t ntt = (size_t)(m + 15) / 16 + 3;  // a launch reads whole groups of up to four tiles
     return type == kTypeQ8_0 ? (size_t)(K / kQK8_0 + 1) / 2 * ntt * kSmPack0 : (size_t)(K / kQKK) * ntt * kSmPackK;

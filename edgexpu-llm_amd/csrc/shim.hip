@@ -59,6 +59,7 @@ hipError_t launch_g32_pack(const float *x, const uint8_t *xq, size_t xq_stride, 
                            hipStream_t st);
 hipError_t launch_gemm_g32(int type, const uint8_t *rw, int n_out, int K, int m, const uint8_t *pack, float *part,
                            unsigned *cnt, const float *bias, float *out, int ldo, hipStream_t st);
+bool gemm_small_take(int type, int n_out, int K, int m);
 size_t gemm_small_pack_bytes(int type, int m, int K);
 hipError_t launch_small_pack(int type, const float *x, const float *y, float eps, int pro, int m, int K,
                              uint8_t *pack, hipStream_t st);
@@ -463,39 +464,17 @@ bool use_exact_gemm(uint32_t type, int nmat, const void *const *w, const int *n_
            exact_gemm_type(type, nmat, w, n_out, n_in, m);
 }
 
-// The few-token GEMM (gemm_small.hip) takes Q4_K (rows of 16-byte vectors),
-// Q6_K and Q8_0 products from kSmallMinTokens tokens: up to 64 always, beyond
-// that while rows x K x (64-token blocks, each of which reads the weights
-// again) stays below the line where the 128-token tiles of the prefill GEMMs
-// catch up.  Measured, few-token / prefill, one matrix: Q4_K 4096 x 4096 of
-// 512 tokens (134 M) 48 / 53 us, 4096 x 14336 of 128 (117 M) 50 / 49, 2560 x
-// 9728 of 256 (100 M) 52 / 48; rows of 8192 and more, whose few tiles the
-// prefill GEMM splits four ways at most: 14336 x 4096 of 192 (176 M) 62 / 84;
-// Q6_K 9728 x 2560 of 192 (75 M) 50 / 60, of 256 (100 M) 70 / 62, 2560 x 2560
-// of 512 (8 blocks, 52 M) 51 / 43; Q8_0 4096 x 4096 of 192 (50 M) 44 / 51, of
-// 256 (67 M) 56 / 52.  Several matrices are one launch here and as many (with
-// a prologue, more) there: gate and up of 2 x 14336 rows of 4096, 131 tokens
-// (352 M) 102 / 119 us, 200 tokens (470 M) 148 / 132.
-constexpr int kSmallMinTokens = 5;
-bool use_small(uint32_t type, int nmat, const void *const *w, const int *n_out, int n_in, int m) {
-    static const int lo = tuning_knob("EXQ_SM_LO", kSmallMinTokens), hi = tuning_knob("EXQ_SM_HI", 0);
-    if (m < lo) return false;
-    if (type != (uint32_t)kTypeQ8_0 && type != (uint32_t)kTypeQ6_K && type != (uint32_t)kTypeQ4_K) return false;
-    const int blocks = (m + 63) / 64;
-    if (hi != 0 ? m > hi : blocks > 1) {
-        if (hi != 0 || blocks > 4096) return false;  // (token blocks are a launch's y dimension)
-        const double limit = type == (uint32_t)kTypeQ4_K   ? (n_in >= 8192 ? 220e6 : 110e6)
-                             : type == (uint32_t)kTypeQ6_K ? 80e6
-                                                           : 56e6;
-        if (type == (uint32_t)kTypeQ6_K && blocks > 5) return false;
-        double rows = 0.0;
-        for (int z = 0; z < nmat; ++z) rows += n_out[z];
-        if (rows * n_in * blocks > limit * (nmat == 1 ? 1.0 : 1.75 * nmat)) return false;
-    }
+// Whether a matrix takes the few-token GEMM: by its own sizes and address
+// alone, so that a group gives the words of its matrices' own calls.
+bool small_matrix(uint32_t type, const void *w, int n_out, int n_in, int m) {
+    if (!gemm_small_take((int)type, n_out, n_in, m)) return false;
     if (type != (uint32_t)kTypeQ4_K) return true;
-    if (m >= gemm_min_tokens(type) && g.prefill_mode != EDGEXPU_HIP_PREFILL_EXACT_INT8) return false;
+    return aligned16(w) && (m < gemm_min_tokens(type) || g.prefill_mode == EDGEXPU_HIP_PREFILL_EXACT_INT8);
+}
+
+bool use_small(uint32_t type, int nmat, const void *const *w, const int *n_out, int n_in, int m) {
     for (int z = 0; z < nmat; ++z)
-        if (!aligned16(w[z])) return false;
+        if (!small_matrix(type, w[z], n_out[z], n_in, m)) return false;
     return true;
 }
 
@@ -692,6 +671,21 @@ bool run_linear_group(uint32_t type, int nmat, const void *const *w, const int *
     }
     if (use_small(type, nmat, w, n_out, n_in, m))
         return run_small(type, nmat, w, n_out, bias, nullptr, out, false, x, nullptr, 0.0f, 0, nullptr, 0, m, n_in, st);
+    if (nmat > 1) {
+        // some of the matrices only: one call for them, one for the others
+        const void *pw[2][4];
+        const float *pb[2][4];
+        float *po[2][4];
+        int pn[2][4], n[2] = {0, 0};
+        for (int z = 0; z < nmat; ++z) {
+            const int k = small_matrix(type, w[z], n_out[z], n_in, m) ? 1 : 0, i = n[k]++;
+            pw[k][i] = w[z], pn[k][i] = n_out[z], po[k][i] = out[z];
+            pb[k][i] = bias != nullptr ? bias[z] : nullptr;
+        }
+        if (n[1] != 0)
+            return run_linear_group(type, n[1], pw[1], pn[1], pb[1], po[1], x, m, n_in, st) &&
+                   run_linear_group(type, n[0], pw[0], pn[0], pb[0], po[0], x, m, n_in, st);
+    }
     // two to four tokens of the rows the streaming GEMV takes are quantized
     // inside its workgroups too; other long rows quantize once in their own
     // launch

@@ -7,6 +7,8 @@ oracle is the order of the f32 sum over blocks), at the edges of the token
 tiles (16), the row tiles (16, 32), the K units (one super-block, one 32-element
 block, counts that do not divide the waves) and the wave counts (1 to 16).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -110,6 +112,63 @@ def test_small_layer_calls_equal_the_steps(hipdev, qt, n_in, n_out, m):
     E.layer_linear([w, w2], qt, x, (n_out, n_out), n_in, residuals=[res, o0], outs=[o0, o1])
     eq(o0, E.add(res, lin(x, w, None)))
     eq(o1, E.add(o0, lin(x, w2, None)))
+
+
+def takes_small(qt, n_out, n_in, m):
+    """The dispatch rule itself (gemm_small_take in csrc/gemm_small.hip)."""
+    f = E.hip().lib._Z15gemm_small_takeiiii
+    f.restype = C.c_bool
+    f.argtypes = [C.c_int] * 4
+    return f(qt, n_out, n_in, m)
+
+
+@pytest.mark.parametrize("qt,n_in,n_outs,m", [(12, 2560, (9728, 1024, 9728), 300), (14, 2560, (9728, 300), 200),
+                                              (8, 2048, (20000, 40), 200)])
+def test_group_equals_each_matrix_across_the_line(hipdev, qt, n_in, n_outs, m):
+    """Past 64 tokens a group may hold matrices on either side of the line to
+    the prefill GEMM: each gives the words of its own call, plain, as a layer
+    call and as a gate / up pair."""
+    taken = [takes_small(qt, n, n_in, m) for n in n_outs]
+    assert True in taken and False in taken
+    rng = np.random.default_rng(qt + m)
+    wd = [dev(synth.np_weights(qt, n, n_in, rng)) for n in n_outs]
+    bd = [dev(rng.normal(0, 0.3, n).astype(np.float32)) for n in n_outs]
+    rd = [dev(rng.normal(0, 3, (m, n)).astype(np.float32)) for n in n_outs]
+    x = dev(synth.np_activations(m, n_in, rng))
+    nw = dev(rng.normal(1, 0.2, n_in).astype(np.float32))
+
+    def eq(a, b, what):
+        assert np.array_equal(bits(a.cpu().numpy()), bits(b.cpu().numpy())), what
+
+    group = E.linear_quant_group(wd, qt, x, list(n_outs), n_in, biases=bd)
+    layer = E.layer_linear(wd, qt, x, list(n_outs), n_in, norm_weight=nw, biases=bd, residuals=rd)
+    for z, n in enumerate(n_outs):
+        eq(group[z], E.linear_quant_batch(wd[z], qt, x, n, n_in, bias=bd[z]), ("group", z))
+        eq(layer[z], E.layer_linear([wd[z]], qt, x, [n], n_in, norm_weight=nw, biases=[bd[z]],
+                                    residuals=[rd[z]])[0], ("layer", z))
+    n = n_outs[0]
+    up = wd[0].flip(0).contiguous()
+    gu = E.linear_quant_group([wd[0], up], qt, x, [n, n], n_in)
+    for z, w in enumerate((wd[0], up)):
+        eq(gu[z], E.linear_quant_batch(w, qt, x, n, n_in), ("pair", z))
+    eq(E.gate_up_silu(wd[0], up, qt, x, n, n_in), E.silu_mul(gu[0], gu[1]), "gate_up_silu")
+
+
+@pytest.mark.parametrize("m", [8, 40])
+def test_group_with_a_matrix_at_another_address(hipdev, m):
+    """Q4_K blocks off a 16-byte address keep to the GEMV; the other matrices
+    of their group give the words of their own calls."""
+    n_out, n_in = 100, 2560
+    rng = np.random.default_rng(m)
+    w = [synth.np_weights(12, n_out, n_in, rng) for _ in range(2)]
+    x = dev(synth.np_activations(m, n_in, rng))
+    off = torch.empty(w[1].size + 16, dtype=torch.uint8, device="cuda:0")
+    off[4:4 + w[1].size] = dev(w[1].reshape(-1))
+    wd = [dev(w[0]), off[4:4 + w[1].size]]
+    group = E.linear_quant_group(wd, 12, x, [n_out, n_out], n_in)
+    for z in range(2):
+        one = E.linear_quant_batch(wd[z], 12, x, n_out, n_in)
+        assert np.array_equal(bits(group[z].cpu().numpy()), bits(one.cpu().numpy())), z
 
 
 @pytest.mark.parametrize("qt,n_in", [(12, 2560), (14, 2560), (8, 576)])
