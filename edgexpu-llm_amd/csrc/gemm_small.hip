@@ -37,6 +37,7 @@
 // with piece {0, 2, 1, 3}[g] (8 bytes) of each 32-byte chunk.  The pack and
 // the Q6_K loads use the same piece order.
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 #include "common.h"
@@ -687,26 +688,40 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_small_kernel(SmallArgs a) {
 using namespace exq;
 
 // True when a matrix of n_out rows of K elements takes this GEMM at m tokens:
-// Q4_K, Q6_K and Q8_0 from kSmallMinTokens tokens, up to 64 always, beyond that
-// while rows x K x (64-token blocks, each of which reads the weights again)
-// stays below the line where the 128-token tiles of the prefill GEMMs catch
-// up.  Measured, few-token / prefill: Q4_K 4096 x 4096 of 512 tokens (134 M)
-// 48 / 53 us, 14336 rows of 4096 at 128 (117 M) 50 / 49, 9728 of 2560 at 256
-// (100 M) 52 / 48; rows of 8192 and more, whose few tiles the prefill GEMM
-// splits four ways at most: 4096 rows of 14336 at 192 (176 M) 62 / 84; Q6_K
-// 2560 rows of 9728 at 192 (75 M) 50 / 60, at 256 (100 M) 70 / 62, 2560 of 2560
-// at 512 (8 blocks, 52 M) 51 / 43; Q8_0 4096 x 4096 of 192 (50 M) 44 / 51, of
-// 256 (67 M) 56 / 52.
+// Q4_K, Q6_K and Q8_0 from kSmallMinTokens tokens.  Up to 64 tokens always
+// (Q4_K to 32), beyond that while rows x K x (64-token blocks, each of which
+// reads the weights again) stays below the line where the 128-token tiles of
+// the prefill GEMMs catch up.  Theirs is one workgroup's walk through K, split
+// four ways at most, whatever the rows: the line rises with K.  Swept over 44
+// shapes of 33 to 768 tokens; nearest the line, few-token / prefill us:
+//   Q4_K 9728 x 2560 (rows x K), 192 tokens (75 M) 42 / 45, 256 (100 M) 51 / 46;
+//     4096 x 4096, 512 (134 M) 47 / 51, 768 (201 M) 66 / 62; 14336 x 4096, 128
+//     (117 M) 49 / 49, 192 (176 M) 69 / 59; 8192 x 8192, 128 (134 M) 48 / 61,
+//     192 (201 M) 68 / 65; 4096 x 14336, 192 (176 M) 69 / 83
+//   Q4_K, one block of 33 to 64 tokens: 32000 x 4096 (131 M) 53 / 61, 28672 x
+//     8192 (235 M) 94 / 89 (48 tokens 81 / 87); 40000 x 2560 (102 M) 54 / 52,
+//     65536 x 2560 (168 M) 83 / 57
+//   Q6_K 2560 x 2560, 384 (39 M) 40 / 40, 448 (46 M) 48 / 42; 4096 x 4096, 192
+//     (50 M) 38 / 45, 256 (67 M) 50 / 47; 2560 x 9728, 192 (75 M) 49 / 58, 256
+//     (100 M) 67 / 62; 4096 x 14336, 128 (117 M) 64 / 84, 256 (235 M) 120 / 108
+//   Q8_0 2560 x 2560, 384 (39 M) 39 / 41, 448 (46 M) 47 / 42; 4096 x 4096, 192
+//     (50 M) 42 / 49, 256 (67 M) 54 / 50; 49152 x 576, 128 (57 M) 66 / 57;
+//     4096 x 14336, 128 (117 M) 87 / 92, 192 (176 M) 125 / 119
+// Below 8 tokens the GEMV is as fast or faster for one matrix of few rows: 5
+// tokens of Q8_0 1024 x 4096 9.8 us there, 11.4 here, 1024 x 28672 37 and 46
+// (of 4096 rows 17 and 12); a group's other matrices would pay for a second
+// quantization.
 constexpr int kSmallMinTokens = 5;
 bool gemm_small_take(int type, int n_out, int K, int m) {
     static const int lo = tuning_knob("EXQ_SM_LO", kSmallMinTokens), hi = tuning_knob("EXQ_SM_HI", 0);
     if ((type != kTypeQ8_0 && type != kTypeQ6_K && type != kTypeQ4_K) || m < lo) return false;
-    const int blocks = (m + 63) / 64;
     if (hi != 0) return m <= hi;
-    if (blocks == 1) return true;
-    if (blocks > 4096 || (type == kTypeQ6_K && blocks > 5)) return false;  // (token blocks are a launch's y dimension)
-    const double limit = type == kTypeQ4_K ? (K >= 8192 ? 220e6 : 110e6) : type == kTypeQ6_K ? 80e6 : 56e6;
-    return (double)n_out * K * blocks <= limit;
+    const int blocks = (m + 63) / 64;
+    if (m <= 32 || (blocks == 1 && type != kTypeQ4_K)) return true;
+    if (blocks > 4096) return false;  // (token blocks are a launch's y dimension)
+    double line = type == kTypeQ4_K ? fmin(25e6 + 27e3 * K, 200e6) : type == kTypeQ6_K ? 20e6 + 7.5e3 * K : 25e6 + 7.5e3 * K;
+    if (blocks == 1) line *= 1.3;  // (its 33 to 64 tokens are 54 on the average)
+    return (double)n_out * K * blocks <= line;
 }
 
 size_t gemm_small_pack_bytes(int type, int m, int K) {
