@@ -216,9 +216,10 @@ __device__ __forceinline__ float reduce_partner(float v, int off) {
 // partners l ^ 32, ^ 16, ..., ^ 1 in that order, each double moved as its
 // two words by reduce_partner (bpermute for ^ 32, swizzles and DPP below),
 // so every lane adds the same pairs in the same order.
+template <int W = 64>
 __device__ __forceinline__ double wave_sum_f64(double s) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
+    for (int off = W / 2; off > 0; off >>= 1) {
         const uint64_t b = __builtin_bit_cast(uint64_t, s);
         const uint32_t lo = __float_as_uint(reduce_partner(__uint_as_float((uint32_t)b), off));
         const uint32_t hi = __float_as_uint(reduce_partner(__uint_as_float((uint32_t)(b >> 32)), off));

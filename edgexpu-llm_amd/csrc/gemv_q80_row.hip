@@ -90,14 +90,20 @@ __global__ __launch_bounds__(kRowThreads) void gemv_q80_row_kernel(RowArgs a) {
     __builtin_amdgcn_sched_barrier(0);
 
     if (PRO == 1) {
-        __shared__ double part[kRowWaves];
-        double s = 0.0;
+        // the fused GEMV's sum, whose thread f holds elements 4 f .. 4 f + 3: this
+        // thread's two such sums, each over 32 lanes here by the partners of its
+        // 64, then their sum
+        __shared__ double part[2 * kRowWaves];
+        double s[2] = {0.0, 0.0};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) s += (double)v[i] * (double)v[i];  // a float square is exact in double
-        s = wave_sum_f64(stages ? s : 0.0);
-        if (lane == 0) part[wave] = s;
+        for (int i = 0; i < 8; ++i) s[i >> 2] += (double)v[i] * (double)v[i];  // a float square is exact in double
+        const double sum = wave_sum_f64<32>(stages ? s[0] : 0.0) + wave_sum_f64<32>(stages ? s[1] : 0.0);
+        if ((lane & 31) == 0) part[threadIdx.x >> 5] = sum;
         __syncthreads();
-        const float scale = rms_scale(((part[0] + part[1]) + part[2]) + part[3], a.nb * kQK8_0, a.eps);
+        double ss = 0.0;
+#pragma unroll
+        for (int w = 0; w < 2 * kRowWaves; ++w) ss += part[w];
+        const float scale = rms_scale(ss, a.nb * kQK8_0, a.eps);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const float t = v[i] * scale;
