@@ -192,6 +192,12 @@ __device__ __forceinline__ float rms_scale(double ss, int n, float eps) {
     return 1.0f / sqrtf(mean + eps);
 }
 
+// The squares of four elements; a float square is exact in double.
+__device__ __forceinline__ double square4(const float4 v) {
+    return ((double)v.x * (double)v.x + (double)v.y * (double)v.y) +
+           ((double)v.z * (double)v.z + (double)v.w * (double)v.w);
+}
+
 __device__ __forceinline__ float shfl_xor_f(float v, int mask) {
     return __shfl_xor(v, mask, 64);
 }

@@ -96,16 +96,29 @@ __device__ __forceinline__ void load8(const float *p, float (&v)[8]) {
     v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
 }
 
-// Sum of squares of the token's row over the workgroup, in double (the wave
-// trees in wave order), then the RMSNorm scale.
-__device__ __forceinline__ float block_rms_scale(double s, int n, float eps) {
-    __shared__ double part[16];
-    s = wave_sum_f64(s);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+// RMSNorm scale of a row of n elements (a multiple of 32) by the workgroup's
+// first 256 threads: the sum of rmsnorm_kernel, term for term, so that a layer
+// call gives the words of its steps.
+constexpr int kRmsThreads = 256;
+__device__ __forceinline__ float row_rms_scale(const float *x, int n, float eps) {
+    __shared__ double part[kRmsThreads / 64];
+    constexpr int kTogether = 4;
+    const float4 *x4 = reinterpret_cast<const float4 *>(x);
+    const int tid = threadIdx.x, n4 = n >> 2;
+    if (tid < kRmsThreads) {
+        double s = 0.0;
+        for (int i0 = tid; i0 < n4; i0 += kTogether * kRmsThreads) {
+            float4 v[kTogether];  // loaded together
+#pragma unroll
+            for (int k = 0; k < kTogether; ++k) v[k] = x4[min(i0 + k * kRmsThreads, n4 - 1)];
+#pragma unroll
+            for (int k = 0; k < kTogether; ++k) s += i0 + k * kRmsThreads < n4 ? square4(v[k]) : 0.0;
+        }
+        s = wave_sum_f64(s);
+        if ((tid & 63) == 0) part[tid >> 6] = s;
+    }
     __syncthreads();
-    double ss = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) ss += part[w];
-    return rms_scale(ss, n, eps);
+    return rms_scale((part[0] + part[1]) + (part[2] + part[3]), n, eps);
 }
 
 __device__ __forceinline__ uint32_t bytes4(const int *q) {
@@ -133,20 +146,7 @@ __global__ __launch_bounds__(1024) void small_pack_k_kernel(const float *__restr
     const float *xr = x + (size_t)t * K;
     const int e0 = 64 * j + 8 * q;
     float scale = 0.0f;
-    if (PRO == 1) {
-        double s = 0.0;
-        for (int sb = first; sb < nsb; sb += per) {
-            float a[8], b[8];
-            load8(xr + sb * kQKK + e0, a);
-            load8(xr + sb * kQKK + e0 + 32, b);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                s += (double)a[i] * (double)a[i];  // a float square is exact in double
-                s += (double)b[i] * (double)b[i];
-            }
-        }
-        scale = block_rms_scale(s, K, eps);
-    }
+    if (PRO == 1) scale = row_rms_scale(xr, K, eps);
     const int last = PRO == 1 ? nsb : min(nsb, ((int)blockIdx.y + 1) * per);
     for (int sb = first; sb < last; sb += per) {
         float xs[16];
@@ -212,16 +212,7 @@ __global__ __launch_bounds__(1024) void small_pack_0_kernel(const float *__restr
     const int K = nb * kQK8_0;
     const float *xr = x + (size_t)t * K;
     float scale = 0.0f;
-    if (PRO == 1) {
-        double s = 0.0;
-        for (int b = first; b < nb; b += per) {
-            float a[8];
-            load8(xr + b * kQK8_0 + 8 * g, a);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s += (double)a[i] * (double)a[i];
-        }
-        scale = block_rms_scale(s, K, eps);
-    }
+    if (PRO == 1) scale = row_rms_scale(xr, K, eps);
     const int last = PRO == 1 ? nb : min(nb, ((int)blockIdx.y + 1) * per);
     for (int b = first; b < last; b += per) {
         float a[8], c[8];
@@ -739,7 +730,7 @@ hipError_t launch_small_pack(int type, const float *x, const float *y, float eps
     int threads = 256;
     if (pro == 1) {
         threads = (nu * lanes + 63) / 64 * 64;
-        threads = threads > 1024 ? 1024 : threads;
+        threads = threads > 1024 ? 1024 : threads < kRmsThreads ? kRmsThreads : threads;
     }
     const dim3 grid((unsigned)m, pro == 1 ? 1u : (unsigned)((nu * lanes + threads - 1) / threads));
     if (q80) {

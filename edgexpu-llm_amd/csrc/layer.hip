@@ -39,10 +39,6 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ 
     const int tid = threadIdx.x, n4 = n >> 2;
     constexpr int kKeep = 4;
     float4 xv[kKeep], wv[kKeep];
-    const auto square = [](const float4 v) {  // a float square is exact in double
-        return ((double)v.x * (double)v.x + (double)v.y * (double)v.y) +
-               ((double)v.z * (double)v.z + (double)v.w * (double)v.w);
-    };
     double s = 0.0;
     if (vec) {
         const float4 *x4 = reinterpret_cast<const float4 *>(xr), *w4 = reinterpret_cast<const float4 *>(w);
@@ -51,8 +47,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ 
 #pragma unroll
         for (int k = 0; k < kKeep; ++k) wv[k] = w4[min(tid + 256 * k, n4 - 1)];
 #pragma unroll
-        for (int k = 0; k < kKeep; ++k) s += tid + 256 * k < n4 ? square(xv[k]) : 0.0;
-        for (int i = tid + 256 * kKeep; i < n4; i += 256) s += square(x4[i]);
+        for (int k = 0; k < kKeep; ++k) s += tid + 256 * k < n4 ? square4(xv[k]) : 0.0;
+        for (int i = tid + 256 * kKeep; i < n4; i += 256) s += square4(x4[i]);
     } else {
         for (int i = tid; i < n; i += 256) {
             const double v = (double)xr[i];

@@ -85,3 +85,19 @@ def test_short_q80_rows_equal_the_fused_gemv(hipdev, n_in):
         few, = E.layer_linear([w[:16]], 8, xd, [16], n_in, norm_weight=nw)
         many, = E.layer_linear([w], 8, xd, [big], n_in, norm_weight=nw)
         assert np.array_equal(bits(few), bits(many[:, :16])), k
+
+
+@pytest.mark.parametrize("qt", [12, 14, 8])
+@pytest.mark.parametrize("n_in", [512, 2048, 8192])
+def test_few_token_layer_calls_equal_rmsnorm_and_product(hipdev, qt, n_in):
+    """RMSNorm in the few-token pack (csrc/gemm_small.hip) and as a call of its own."""
+    rng = np.random.default_rng(qt + n_in)
+    m, n_out = 6, 48
+    w = dev(synth.np_weights(qt, n_out, n_in, rng))
+    for k in range(20):
+        rows = [steered_row(rng, n_in) for _ in range(m)]
+        x = dev(np.stack([r[0] for r in rows]))
+        nw = dev(telling_weights(rng, *rows[0]) if qt == 8 else rng.uniform(0.9, 1.1, n_in).astype(F))
+        layer, = E.layer_linear([w], qt, x, [n_out], n_in, norm_weight=nw, eps=float(EPS))
+        steps = E.linear_quant_batch(w, qt, E.rmsnorm(x, nw, float(EPS)), n_out, n_in)
+        assert np.array_equal(bits(layer), bits(steps)), k
