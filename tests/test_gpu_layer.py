@@ -48,6 +48,34 @@ def test_rmsnorm_bit_exact(hipdev, ora, n, m, eps):
     assert np.array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("n", [1, 3, 63, 101, 577, 4099])
+def test_rmsnorm_rows_of_any_length(hipdev, ora, n):
+    """Rows that are no whole float4s are read element by element."""
+    rng = np.random.default_rng(n)
+    x, w = rows(rng, 5, n), rng.normal(1, 0.2, n).astype(np.float32)
+    got = E.rmsnorm(dev(x), dev(w), 1e-5).cpu().numpy()
+    assert np.array_equal(bits(got), bits(ora.rmsnorm(x, w, 1e-5)))
+
+
+@pytest.mark.parametrize("n", [256, 4096, 4100])
+@pytest.mark.parametrize("off", ["x", "w", "out"])
+def test_rmsnorm_at_any_float_address(hipdev, ora, n, off):
+    """One pointer off a 16-byte address: the same rows, and nothing past them written."""
+    rng = np.random.default_rng(n)
+    x, w = rows(rng, 3, n), rng.normal(1, 0.2, n).astype(np.float32)
+    at = {}
+    for name, a in (("x", x), ("w", w), ("out", np.full_like(x, 7.0))):
+        k = 1 if name == off else 0
+        buf = torch.full((a.size + 8,), 7.0, device="cuda:0")
+        buf[k:k + a.size] = dev(a.reshape(-1))
+        at[name] = buf[k:k + a.size].view(a.shape)
+        if name == "out":
+            tail = buf[k + a.size:]
+    E.rmsnorm(at["x"], at["w"], 1e-5, out=at["out"])
+    assert np.array_equal(bits(at["out"].cpu().numpy()), bits(ora.rmsnorm(x, w, 1e-5)))
+    assert bool((tail == 7.0).all())
+
+
 def test_rmsnorm_edge_rows(hipdev, ora):
     """All-zero row (scale 1/sqrt(eps)), a single nonzero, in-place call."""
     n = 4096

@@ -251,8 +251,8 @@ def test_prefill_gemm_vs_oracle(hipdev, ora, n_in, n_out, m):
     """m >= 16 Q4_K products run on the matrix cores with exact block integers;
     every output within the fp32 bound of the reference (oracle) on its
     conditioning scale.  Shapes cover ragged token and row counts, one
-    super-block, the K range split in two (odd super-block count 5 included)
-    and unsplit (129 row blocks)."""
+    super-block, an odd super-block count and 16385 rows.  (These sizes take the
+    few-token GEMM; test_gpu_prefill.py has the prefill GEMM's.)"""
     rng = np.random.default_rng(900 + n_in + n_out + m)
     w = synth.np_weights(12, n_out, n_in, rng)
     x = synth.np_activations(m, n_in, rng)
@@ -332,7 +332,7 @@ def test_odd_weight_addresses_are_refused(hipdev, qt):
 
 @pytest.mark.parametrize("n_in,n_out", [(4096, 4096), (4096, 14336), (14336, 4096)])
 def test_prefill_gemm_full_shape(hipdev, ora, n_in, n_out):
-    """The three prefill shapes at m = 512 against the float64 restatement
+    """Three layer shapes at m = 512 (the two of 14336 on the prefill GEMM) against the float64 restatement
     (exact integers, float64 combine); a row sample also against the oracle."""
     m = 512
     rng = np.random.default_rng(77 + n_in + n_out)
@@ -352,12 +352,13 @@ def test_prefill_gemm_full_shape(hipdev, ora, n_in, n_out):
 @pytest.mark.parametrize("n_in,n_out,m", [(2560, 300, 16), (4096, 257, 64), (256, 70, 129), (9728, 130, 100),
                                           (1280, 515, 200), (2048, 384, 512), (1024, 16385, 33), (512, 129, 47)])
 def test_prefill_gemm_kq_vs_oracle(hipdev, ora, qt, n_in, n_out, m):
-    """Q6_K products from 16 tokens and Q5_K from 32 run on the matrix cores
-    over a per-call repack, two exact chains per K-step (scale split
-    16 s1 + s0; Q5_K at 16 tokens takes the GEMV); every
-    output within the fp32 bound of the oracle on its conditioning scale.
-    Shapes cover one super-block, ragged tokens and rows, the K split (odd
-    super-block counts), 129 row blocks and a full 512-token block."""
+    """Q5_K products from 32 tokens run on the matrix cores over a per-call
+    repack, two exact chains per K-step (scale split 16 s1 + s0; at 16 tokens
+    they take the GEMV); every output within the fp32 bound of the oracle on its
+    conditioning scale.  Shapes cover one super-block, ragged tokens and rows,
+    the K split (odd super-block counts), 129 row blocks and a full 512-token
+    block.  Q6_K at these sizes is the few-token GEMM (test_gpu_prefill.py has
+    the repacked one's)."""
     rng = np.random.default_rng(4100 + 7 * qt + n_in + n_out + m)
     w = synth.np_weights(qt, n_out, n_in, rng)
     x = synth.np_activations(m, n_in, rng)
@@ -371,7 +372,7 @@ def test_prefill_gemm_kq_vs_oracle(hipdev, ora, qt, n_in, n_out, m):
 
 @pytest.mark.parametrize("qt", [13, 14])
 def test_prefill_gemm_kq_from_q8k(hipdev, ora, qt):
-    """The same GEMM fed with Q8_K blocks already in memory (the activation
+    """The same products fed with Q8_K blocks already in memory (the activation
     pack built from the blocks, not from f32 rows): identical to the f32 entry."""
     n_in, n_out, m = 2304, 200, 40
     rng = np.random.default_rng(4400 + qt)
@@ -439,12 +440,13 @@ def _q80_rows(ora, x):
 @pytest.mark.parametrize("n_in,n_out,m", [(576, 1536, 16), (1536, 576, 64), (4096, 257, 100), (96, 70, 129),
                                           (2048, 300, 512), (1024, 16385, 33), (160, 129, 47), (14336, 130, 20)])
 def test_prefill_gemm_g32_vs_oracle(hipdev, ora, qt, n_in, n_out, m):
-    """m >= 16 Q8_0 / Q4_0 / Q5_0 products run on the matrix cores over a
-    per-call repack into 128-element records, one exact chain per block and
-    a per-block combine; every output within the fp32 bound of the oracle on
-    its conditioning scale.  Shapes: the 576 / 1536 hidden sizes, rows that
-    end inside a record (96, 160, 576), the K split, 129 row blocks, a full
-    512-token block."""
+    """m >= 16 Q4_0 / Q5_0 products run on the matrix cores over a per-call
+    repack into 128-element records, one exact chain per block and a per-block
+    combine; every output within the fp32 bound of the oracle on its
+    conditioning scale.  Shapes: the 576 / 1536 hidden sizes, rows that end
+    inside a record (96, 160, 576), the K split, 129 row blocks, a full
+    512-token block.  Q8_0 at these sizes is the few-token GEMM
+    (test_gpu_prefill.py has the repacked one's)."""
     rng = np.random.default_rng(4700 + 11 * qt + n_in + n_out + m)
     w = synth.np_weights(qt, n_out, n_in, rng)
     x = synth.np_activations(m, n_in, rng)
@@ -458,7 +460,7 @@ def test_prefill_gemm_g32_vs_oracle(hipdev, ora, qt, n_in, n_out, m):
 
 @pytest.mark.parametrize("qt", [8, 2, 6])
 def test_prefill_gemm_g32_from_q80(hipdev, ora, qt):
-    """The same GEMM fed with Q8_0 blocks already in memory: identical to the
+    """The same products fed with Q8_0 blocks already in memory: identical to the
     f32 entry (the packer's quantization is the Q8_0 quantizer's)."""
     n_in, n_out, m = 1248, 200, 40
     rng = np.random.default_rng(4800 + qt)
@@ -496,7 +498,8 @@ def test_prefill_gemm_g32_integers_exact(hipdev, qt):
 
 @pytest.mark.parametrize("n_in,n_out", [(576, 1536), (4096, 4096)])
 def test_prefill_gemm_q80_full_shape(hipdev, ora, n_in, n_out):
-    """Q8_0 at m = 512: a row sample against the float64 restatement, a token
+    """Q8_0 at m = 512 (576 x 1536 on the few-token GEMM, 4096 x 4096 on the
+    prefill GEMM): a row sample against the float64 restatement, a token
     sample also against the oracle."""
     m = 512
     rng = np.random.default_rng(5000 + n_in)
@@ -623,8 +626,8 @@ def test_prefill_gemm_integers_exact(hipdev, n_in, n_out, m):
     """Unit scales (d = dmin = 1) and integer activations that are their own
     Q8_K codes (each block's first element -127: d = 1): every fp32 step of the
     GEMM is then exact, so the output equals the int64 closed form exactly --
-    the block integers are exact through the matrix cores, with the K range
-    split in two (2 tiles) and unsplit (132 tiles)."""
+    the block integers are exact through the matrix cores (of the few-token GEMM
+    at these sizes; test_gpu_prefill.py has the prefill GEMM's)."""
     rng = np.random.default_rng(5150 + n_out)
     w = _q4k_headers(synth.np_weights(12, n_out, n_in, rng), 1.0, 1.0)
     x = rng.integers(-127, 128, (m, n_in)).astype(np.float32)
@@ -637,11 +640,11 @@ def test_prefill_gemm_integers_exact(hipdev, n_in, n_out, m):
 
 
 def test_prefill_gemm_two_chains(hipdev, ora):
-    """Tokens whose Q8_K codes are all +-127 (sum |q8| = 32512 per super-block,
-    beyond the 17753 one exact chain allows) run every super-block as two
-    chains; rows with every scale and min 63 and every code 15 push sumi to
-    30.7 M.  Mixed with ordinary tokens in other workgroups' token blocks.
-    Outputs within the bound of the float64 restatement and of the oracle."""
+    """Tokens whose Q8_K codes are all +-127 (sum |q8| = 32512 per super-block)
+    and rows with every scale and min 63 and every code 15, which push sumi to
+    30.7 M: beyond one exact fp16 chain of the prefill GEMM (test_gpu_prefill.py),
+    and here the largest integers of the few-token GEMM.  Mixed with ordinary
+    tokens.  Outputs within the bound of the float64 restatement and of the oracle."""
     rng = np.random.default_rng(6161)
     n_in, n_out, m = 2048, 300, 200
     w = synth.np_weights(12, n_out, n_in, rng)
@@ -659,19 +662,8 @@ def test_prefill_gemm_two_chains(hipdev, ora):
     assert_tol(got[:4], want, S[:4], "two chains vs oracle")
 
 
-@pytest.mark.parametrize("qt", [12, 13, 14])
-def test_prefill_pack_special_blocks(hipdev, ora, qt):
-    """The f32 activation pack of the K-quant prefill GEMMs (four tokens per
-    wavefront) quantizes as the reference's quantize_row_q8_K does
-    (src/gguf_dot_q8.c:360-412) up to the sign of a block's codes and scale,
-    which cancels in the GEMM: the GEMM over it equals, bit for bit, the GEMM
-    over the oracle's Q8_K bytes of the same activations.  Blocks: all
-    zero, the largest magnitude twice with opposite signs (negative first,
-    positive first, in one lane and in lanes far apart), NaN elements, -0.0
-    and subnormals, codes at exact .5 ties, a block whose maximum is its last
-    element, and a token count that leaves a wavefront's last tokens past m."""
-    rng = np.random.default_rng(4242 + qt)
-    n_in, n_out, m = 1024, 96, 37
+def special_blocks(m, n_in, rng):
+    """Activations whose first nine tokens hold the blocks a Q8_K quantizer can go wrong on (n_in >= 1024)."""
     x = synth.np_activations(m, n_in, rng)
     x[0, 0:256] = 0.0                                   # all-zero block
     x[1, 256:512] = -0.0
@@ -691,7 +683,24 @@ def test_prefill_pack_special_blocks(hipdev, ora, qt):
     x[7, 512:768] = 0.0
     x[7, 512 + 100] = -7.0                              # one element, negative
     x[8, 768:1024] = x[8, 768:1024] * 1e6
-    x = x.astype(np.float32)
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("qt", [12, 13, 14])
+def test_prefill_pack_special_blocks(hipdev, ora, qt):
+    """The f32 activation packs of the K-quant GEMMs (Q5_K: the prefill GEMM's,
+    four tokens per wavefront; Q4_K, Q6_K: the few-token GEMM's, 16 lanes a
+    super-block) quantize as the reference's quantize_row_q8_K does
+    (src/gguf_dot_q8.c:360-412) up to the sign of a block's codes and scale,
+    which cancels in the GEMM: the GEMM over it equals, bit for bit, the GEMM
+    over the oracle's Q8_K bytes of the same activations.  Blocks: all
+    zero, the largest magnitude twice with opposite signs (negative first,
+    positive first, in one lane and in lanes far apart), NaN elements, -0.0
+    and subnormals, codes at exact .5 ties, a block whose maximum is its last
+    element, and a token count that leaves a wavefront's last tokens past m."""
+    rng = np.random.default_rng(4242 + qt)
+    n_in, n_out, m = 1024, 96, 37
+    x = special_blocks(m, n_in, rng)
     w = synth.np_weights(qt, n_out, n_in, rng)
     bias = rng.normal(0, 0.5, n_out).astype(np.float32)
     got = E.linear_quant_batch(dev(w), qt, dev(x), n_out, n_in, bias=dev(bias)).cpu().numpy()
@@ -707,8 +716,8 @@ def test_prefill_pack_special_blocks(hipdev, ora, qt):
 def test_prefill_gemm_q8k_input_and_repeat(hipdev, ora):
     """The GEMM over Q8_K block bytes already in memory (edgexpu_hip_gemv_q8_dev)
     equals the GEMM over the f32 activations bit for bit (same codes, same
-    operand pack), and a second call gives the same bits (the split-K flags
-    the first call used are back at zero)."""
+    operand pack), and a second call gives the same bits (test_gpu_prefill.py
+    has the same past the few-token GEMM, where the K split counts arrivals)."""
     rng = np.random.default_rng(7272)
     n_in, n_out, m = 4096, 300, 100
     w = synth.np_weights(12, n_out, n_in, rng)
