@@ -302,8 +302,8 @@ hipError_t launch_gemv_fused_layer(int type, int nmat, const uint8_t *const *w, 
         return hipErrorInvalidValue;
     // Q4_K rows at the decode lengths: the streaming kernel (one token: every
     // variant -- plain, prologues, residual, pairs, staged or Q8_K input;
-    // two to four tokens: plain projections of staged tokens), and staged
-    // tokens of Q6_K rows of 9728; its rows equal this kernel's bit for bit
+    // two to four staged tokens: projections, plain or with a residual), and
+    // staged tokens of Q6_K rows of 9728; its rows equal this kernel's bit for bit
     long long rows = 0;
     for (int z = 0; z < nmat; ++z) rows += n_out[z];
     // few Q8_0 rows, same words as below in a shorter launch
@@ -311,6 +311,7 @@ hipError_t launch_gemv_fused_layer(int type, int nmat, const uint8_t *const *w, 
         return launch_gemv_q80_row(nmat, w, n_out, bias, resid, out, K, x, x2, nw, eps, pro, pair, st);
     if (gemv_stream_take(type, K, m, rows, nmat, w, code, x != nullptr))
         return launch_gemv_stream(type, nmat, w, n_out, bias, resid, out, K, m, x, xq, x2, nw, eps, pro, pair, st);
+    if (m != 1 && code != 0) return hipErrorInvalidValue;
     a.nblk = q8_0_family(type) ? K / kQK8_0 : K / kQKK;
     a.U = q8_0_family(type) ? a.nblk : a.nblk * 4;
     // three waves per row: one-token K-quant launches (Q4_K, Q6_K)

@@ -995,7 +995,7 @@ hipError_t launch_stream_q6k(int fl, const StreamArgs &a, hipStream_t st) {
     }
 }
 
-// Plain projections of m = 2..4 staged tokens.  Rows of 4096 in launches
+// Projections of m = 2..4 staged tokens, plain or (FL) with a residual.  Rows of 4096 in launches
 // of at most three steps per wave keep one row per wave in flight (measured,
 // q+k+v [6144 x 4096] at 2 / 3 / 4 tokens: 6.5 / 7.9 / 8.5 us, against 7.3 /
 // 8.1 / 9.1 with two slots filled twice at the start; o [4096 x 4096] 5.7 /
