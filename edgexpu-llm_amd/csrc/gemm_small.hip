@@ -4,7 +4,10 @@
 // as they lie, up to four matrices of one input in a launch, or a gate / up
 // pair that leaves as silu(gate) * up.
 //
-// What bounds it: the weights, read once per 64 tokens.  The 8-token GEMV
+// What bounds it: not yet the weights, read once per 64 tokens, but waits on
+// memory with few waves (counted on layers of 8 and 45 tokens: waves wait 42-72 %
+// of their time, VALU 13-31 % and MFMA 3-10 % busy, 1 to 2.6 waves a SIMD).  The
+// 8-token GEMV
 // this replaces dots every weight byte with every token on the VALU; the
 // 128-token GEMM tiles leave most of the chip idle on these sizes and add the
 // K split's partial tiles through memory.  Here a workgroup owns 16 (or 32)

@@ -104,11 +104,13 @@ namespace {
 
 constexpr int kGemvMaxTokens = 8;
 constexpr int kFusedMaxTokens = 4;
-// From 16 tokens the matrix-core GEMM reads each weight row once for all
-// tokens; below that the GEMV reads it once per 8 tokens.  Measured at
-// [14336 x 4096] Q4_K: GEMV 44 / 80 / 151 us at 8 / 16 / 32 tokens, GEMM
-// 40 / 41 / 46 us at 16 / 32 / 64 ([4096 x 4096]: GEMV 18 / 31 / 55, GEMM
-// 29 / 31 / 35).  Q5_K pays a weight repack per call: GEMV 31 / 55 us at 16 /
+// From 16 tokens the prefill GEMMs read each weight row once for all tokens;
+// below that the GEMV reads it once per 8 tokens.  (Q4_K, Q6_K and Q8_0 take
+// the few-token GEMM from 5 tokens up to its line, gemm_small_take; these are
+// for what it leaves: the other formats, unaligned Q4_K blocks, matrices past
+// the line.)  Measured at [14336 x 4096] Q4_K: GEMV 44 / 80 / 151 us at 8 / 16 /
+// 32 tokens, GEMM 40 / 41 / 46 us at 16 / 32 / 64 ([4096 x 4096]: GEMV 18 / 31 /
+// 55, GEMM 29 / 31 / 35).  Q5_K pays a weight repack per call: GEMV 31 / 55 us at 16 /
 // 32 tokens against 47 / 48, so it switches at 32.
 constexpr int kPrefillTokens = 16;
 int gemm_min_tokens(uint32_t type) { return type == (uint32_t)kTypeQ5_K ? 32 : kPrefillTokens; }

@@ -72,10 +72,10 @@ int edgexpu_hip_set_prefill_mode(int mode);
 int edgexpu_hip_prefill_mode(void);
 /* Decode GEMV kernel for the launches both kernels cover: one token of Q4_K
  * rows of 2560, 4096 or 14336 elements or of Q6_K rows of 9728 (every
- * variant), plain projections of 2-4 tokens of those rows (activations
- * given as f32), and the f32-activation logits of one or two tokens against
- * Q4_K rows of 4096 or Q6_K rows of 2560.  No reference counterpart (the
- * reference has one CPU kernel).
+ * variant), projections of 2-4 tokens of those rows, plain or with a
+ * residual (activations given as f32), and the f32-activation logits of one
+ * or two tokens against Q4_K rows of 4096 or Q6_K rows of 2560.  No reference
+ * counterpart (the reference has one CPU kernel).
  *  EDGEXPU_HIP_GEMV_AUTO (default): the streaming kernel (weight rows
  *    through LDS by DMA), except launches of fewer than 2048 rows of 9728
  *    Q6_K elements or of 14336 Q4_K elements at 1-3 tokens, which take the
@@ -136,7 +136,16 @@ int edgexpu_hip_weight_n_in(const edgexpu_hip_weight *w);
  * GGUF tensors in a device copy of a file's data section always qualify.
  * Blocks at 16-byte addresses can take the streaming GEMV and logits (Q4_K,
  * Q6_K) and the matrix-core products (Q4_K; the others need even addresses);
- * blocks elsewhere take the fused GEMV, with the same results. ---- */
+ * blocks elsewhere take the fused or generic GEMV: up to four tokens (of
+ * 14336 elements: three) and in the logits with the same results, beyond that
+ * in another summation order (both within 1e-5 of each row's conditioning
+ * scale of the reference).
+ *
+ * Under graph capture: a captured call whose matrices all take the few-token
+ * GEMM (Q4_K, Q6_K and Q8_0 from 5 tokens, see edgexpu_hip_layer_linear_dev)
+ * stays valid until edgexpu_hip_shutdown whatever calls come after it, and
+ * needs no call before it.  The other paths' workspaces are freed when a later
+ * call needs a larger one: capture over them after the largest call. ---- */
 
 /* out[t*n_out + o] = bias[o] + dot(W[o], q8(x[t]))  for t < m.
  * Replaces edgexpu_cpu_linear_quant_batch (include/edgexpu/cpu_kernel.h:71-80,
@@ -153,7 +162,9 @@ int edgexpu_hip_linear_quant_batch_dev(float *out, const float *x, const void *w
  * out[z][t*n_out[z] + o] = bias[z][o] + dot(W_z[o], q8(x[t])) for z < nmat
  * (1..4).  All matrices share type and n_in; bias may be NULL or hold NULL
  * entries.  Equivalent to nmat edgexpu_hip_linear_quant_batch_dev calls
- * (src/native.c:2530-2532 and :2576-2577 issue them back to back). */
+ * (src/native.c:2530-2532 and :2576-2577 issue them back to back), bit for
+ * bit where all blocks start at 16-byte addresses: from 5 tokens a matrix takes
+ * the kernel of its own sizes, in as many launches as that needs. */
 int edgexpu_hip_linear_quant_group_dev(int nmat, float *const *out, const float *x, const void *const *w,
                                        uint32_t type, const float *const *bias, const int *n_out, int m, int n_in,
                                        void *stream);
@@ -278,9 +289,16 @@ int edgexpu_hip_silu_mul_dev(float *out, const float *gate, const float *up, lon
  * edgexpu_cpu_linear_quant_batch (include/edgexpu/cpu_kernel.h:60-80), then
  * edgexpu_cpu_add compute it: the same result as those entry points of this
  * library in sequence (the layer ops above, edgexpu_hip_linear_quant_group_dev).
+ * (one token's RMSNorm sums its squares in another order than
+ * edgexpu_hip_rmsnorm_dev; from two tokens on the order is that call's).
  * One token with the prologue, or no prologue, runs as one launch (the
- * prologue in the GEMV's activation staging, the residual in its store);
- * other shapes run the same steps as separate launches.  out[z] may be
+ * prologue in the GEMV's activation staging, the residual in its store), and
+ * so do two to four tokens with a residual alone of the rows the streaming
+ * kernel takes.  From 5 tokens Q4_K (at 16-byte addresses), Q6_K and Q8_0
+ * matrices up to a size that falls with the tokens take the few-token GEMM: a
+ * pack launch with the prologue, a product launch with the residual.  Other
+ * shapes, and outputs that overlap a residual or bias of the call still to be
+ * read, run the same steps as separate launches.  out[z] may be
  * residual[z] (an in-place residual update); out must not overlap x or x2.
  * x, x2, norm_weight 16-byte aligned.  Returns 1 on success, 0 on bad
  * arguments or a HIP error. */
@@ -294,7 +312,8 @@ int edgexpu_hip_layer_linear_dev(int nmat, float *const *out, const float *x, co
  *   a   = rmsnorm(x; norm_weight, eps)  (norm_weight != NULL) or x
  *   act = silu(b_gate + W_gate . q8(a)) * (b_up + W_up . q8(a))   [m][n_ff]
  * as edgexpu_hip_layer_linear_dev over gate and up followed by
- * edgexpu_hip_silu_mul_dev compute it (bit for bit).  At one token it is one
+ * edgexpu_hip_silu_mul_dev compute it (bit for bit).  From 5 tokens matrices
+ * of the few-token GEMM take its two launches.  At one token it is one
  * launch: row j of gate and row j of up are reduced in the same wave and the
  * store writes their product, so SiLU runs once per element and the down
  * projection takes act with no prologue.  Biases optional; act must not
